@@ -29,6 +29,8 @@ SIGNATURES = {
     "convrot_prepare_modulated": (_i32, [_vp, _i32, _i64, _i64, _i32, _i32, _vp, _vp, _i64, ctypes.c_float, _vp,
                                          _vp, _vp]),
     "convrot_prepare_gelu": (_i32, [_vp, _i64, _i64, _vp, _i64, _i64, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
+    "convrot_linear_rows": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _i64,
+                                   _vp, _vp]),
     "convrot_w4a4_gemm": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i32, _vp]),
     "convrot_w4a4_gemm_residual": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _i64,
                                           _vp, _i32, _vp]),
@@ -141,7 +143,8 @@ def set_tuning(name: str, value: str | None) -> None:
     restores the automatic choice.  Names: gemm_tile ("BMxBN[wWMxWN[sS]]"), gemm_sk (0/1),
     gemm_sk_min, gemm_no_dma, gemm_smallm_max, w4a4_smallm_cfg (A/B/C/F), w4a16_cfg
     (A/B/C/D/E/F, S: split K, T), w4a16_tile ("BMxBN"), prep_ni (1/3/4), sk_spin_limit, gemm_persist (0: never;
-    G: always, on G workgroups), gemm_mfma32 (0/1), fp6_tile ("BMxBN": 256x256, 256x224, 128x256, 128x192, 128x128)."""
+    G: always, on G workgroups), gemm_mfma32 (0/1), fp6_tile ("BMxBN": 256x256, 256x224, 128x256, 128x192, 128x128),
+    linear_rows_cfg (1/2/3/5/16)."""
     check(load().convrot_set_tuning(name.encode(), None if value is None else str(value).encode()))
 
 

@@ -859,6 +859,54 @@ def hip_w4a16_matmul(activations, qweight, wscales, bias, *, output_dtype, out_f
     return out
 
 
+# ------------------------------------------------------------------ few rows
+#
+# convrot_linear_rows runs a layer's preparation inside its GEMM, one launch
+# instead of two: a call of a few rows is launches and latency.  Every workgroup
+# repeats the preparation, ~0.8 us a row of 3072 features, so the rows are
+# bounded: a single row of any length the kernel takes, and more as long as they
+# cost less than the second launch.  HIP-graph replays, two launches -> one, bf16:
+# W4A4 at K = 3072, M = 2: 6.5 -> 5.8 us (N = 3072), 12.8 -> 10.1 (18432); M = 3:
+# 6.55 -> 6.73, 13.1 -> 10.9; K = 1024 -> 1536, M = 4: 5.1 -> 4.8, M = 6: 5.1 -> 5.5.
+# W4A16 (no codes): K = 3072, M = 4: 7.2 -> 6.6, 13.5 -> 12.1; K = 1024, M = 8:
+# 6.0 -> 4.5; K = 8192, M = 2: 8.9 -> 9.3.  An eager call also saves ~8 us of host
+# work (a launch and two buffers).
+LINEAR_ROWS_MAX = {True: (4, 6144), False: (8, 12288)}  # W4A4, W4A16: rows, elements of x
+LINEAR_ROWS_MAX_BYTES = 32768  # of x, include/convrot_amd.h
+LINEAR_ROWS_GROUPS = (64, 256)
+
+
+def _linear_rows_eligible(x2d: torch.Tensor, group_size: int, a4: bool) -> bool:
+    """Whether ConvRotLinear runs these rows through convrot_linear_rows."""
+    rows, features = x2d.shape
+    max_rows, max_elements = LINEAR_ROWS_MAX[a4]
+    return (group_size in LINEAR_ROWS_GROUPS
+            and (rows == 1 or (1 < rows <= max_rows and rows * features <= max_elements))
+            and x2d.dtype in ((torch.bfloat16, torch.float16, torch.float32) if a4
+                              else (torch.bfloat16, torch.float16))
+            and rows * features * x2d.element_size() <= LINEAR_ROWS_MAX_BYTES)
+
+
+def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, wscales, bias, n: int,
+                 gr: GatedResidual | None) -> torch.Tensor:
+    """The whole layer on a few rows: `w` its CDNA4 weight, `gr` a residual that is not in place."""
+    m, k = x2d.shape
+    _validate_mpp_epilogue(m, n, None, wscales, bias)
+    device = nat.require_device(x2d, w, wscales, bias)
+    x2d, w = x2d.contiguous(), w.contiguous()
+    ws, b = _f32(wscales), _f32(bias)
+    out = torch.empty((m, n), dtype=x2d.dtype, device=device)
+    nat.check(
+        nat.load().convrot_linear_rows(
+            nat.ptr(x2d), nat.dtype_code(x2d.dtype), group_size, int(a4), nat.ptr(w), nat.ptr(ws), nat.ptr(b), m, n,
+            k, nat.ptr(gr.residual if gr is not None else None), nat.ptr(gr.gate if gr is not None else None),
+            gr.stride if gr is not None else 0, gr.rows_per_gate if gr is not None else 1, nat.ptr(out),
+            nat.stream_of(device),
+        )
+    )
+    return out
+
+
 # Reference names (the reference's Metal/MPP entry points) -> the gfx950 kernels.
 metal_fused_prepare_convrot_activation = hip_fused_prepare_convrot_activation
 metal_fused_prepare_convrot_activation_i8 = hip_fused_prepare_convrot_activation_i8
@@ -1038,6 +1086,14 @@ class ConvRotLinear(nn.Module):
         if x.shape[-1] != self.in_features:
             raise ValueError(f"ConvRotLinear expected K={self.in_features}, got {x.shape[-1]}")
         x2d = x.reshape(-1, self.in_features)
+        # in place, the output may be x itself, which every workgroup of the one launch reads
+        if not inplace and (gate is None or residual is not None) and _linear_rows_eligible(x2d, self.group_size,
+                                                                                            self.a4):
+            out_shape = (*x.shape[:-1], self.out_features)
+            w = self._device_weight()
+            gr = None if residual is None else _gated_residual(residual, gate, out_shape, x.dtype)
+            return _linear_rows(x2d, self.group_size, self.a4, w, self.scales, self.bias, self.out_features,
+                                gr).reshape(out_shape)
         return self._project(lambda mode: _prepare(x2d, self.group_size, mode), x.shape[:-1], x.dtype,
                              residual, gate, inplace)
 

@@ -97,7 +97,7 @@ int convrot_set_tuning(const char* name, const char* value) {
                 {"w4a16_cfg", kTuneW4a16Cfg},         {"w4a16_tile", kTuneW4a16Tile},
                 {"prep_ni", kTunePrepNi},             {"sk_spin_limit", kTuneSkSpinLimit},
                 {"gemm_persist", kTuneGemmPersist},   {"gemm_mfma32", kTuneGemmMfma32},
-                {"fp6_tile", kTuneFp6Tile}};
+                {"fp6_tile", kTuneFp6Tile},           {"linear_rows_cfg", kTuneRowsCfg}};
   int key = -1;
   for (const auto& n : kNames)
     if (strcmp(n.name, name) == 0) key = n.key;
@@ -130,6 +130,10 @@ int convrot_set_tuning(const char* name, const char* value) {
       case kTuneW4a16Cfg:
         good = strchr("ABCDEFST", value[0]) != nullptr && value[1] == '\0';
         v = value[0];
+        break;
+      case kTuneRowsCfg:
+        v = atoi(value);
+        good = v == 1 || v == 2 || v == 3 || v == 5 || v == 16;
         break;
       default: {
         char* end = nullptr;
@@ -556,6 +560,45 @@ int convrot_w4a16_gemm_ws(const void* act, int act_dtype, const uint8_t* qweight
   return launch_status(convrot::launch_w4a16_gemm(act, act_dtype, qweight, wscales, bias, M, N, K, out, out_dtype,
                                                   (hipStream_t)stream, gr, work),
                        "convrot_w4a16_gemm_ws");
+}
+
+int convrot_linear_rows(const void* x, int dtype, int group_size, int a4, const uint8_t* qweight,
+                        const float* wscales, const float* bias, int64_t M, int64_t N, int64_t K,
+                        const void* residual, const void* gate, int64_t gate_stride, int64_t rows_per_gate, void* out,
+                        void* stream) {
+  if (!valid_dtype(dtype)) return fail(CONVROT_ERR_INVALID, "unsupported activation dtype code %d", dtype);
+  if (M < 0 || N < 0 || K <= 0)
+    return fail(CONVROT_ERR_INVALID, "invalid shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+  const int s = log4_group(group_size);
+  if (s < 0) return fail(CONVROT_ERR_INVALID, "Regular Hadamard size must be a power of 4, got %d", group_size);
+  if (K % group_size)
+    return fail(CONVROT_ERR_INVALID, "features %lld not divisible by ConvRot group size %d", (long long)K, group_size);
+  if (N > 0x7fffffff || packed_weight_bytes(N, K) >= kMaxWeightBytes)
+    return fail(CONVROT_ERR_UNSUPPORTED, "packed weights are limited to 2 GiB (N=%lld K=%lld)", (long long)N,
+                (long long)K);
+  if (gate && !residual) return fail(CONVROT_ERR_INVALID, "a gate needs a residual");
+  if (gate && rows_per_gate <= 0)
+    return fail(CONVROT_ERR_INVALID, "rows_per_gate must be positive, got %lld", (long long)rows_per_gate);
+  if (M == 0 || N == 0) return ok();
+  if (!convrot::linear_rows_eligible(M, K, dtype, s, a4 != 0))
+    return fail(CONVROT_ERR_UNSUPPORTED,
+                "the few-row linear takes 1 to 16 rows of at most 32 KB in all, groups of 64 or 256 and (W4A16) "
+                "16-bit activations; got M=%lld K=%lld group %d %s",
+                (long long)M, (long long)K, group_size, dtype_name(dtype));
+  if (!x || !qweight || !wscales || !out) return fail(CONVROT_ERR_INVALID, "null pointer argument");
+  if (!aligned(x, 16) || !aligned(qweight, 16) || !aligned(out, 16))
+    return fail(CONVROT_ERR_INVALID, "x, qweight and out must be 16-byte aligned");
+  // every workgroup reads all of x, so no workgroup may write into it
+  const int64_t esize = dtype == CONVROT_DTYPE_F32 ? 4 : 2;
+  const uintptr_t xa = (uintptr_t)x, oa = (uintptr_t)out;
+  if (xa < oa + (uintptr_t)(M * N * esize) && oa < xa + (uintptr_t)(M * K * esize))
+    return fail(CONVROT_ERR_INVALID, "out must not overlap x");
+  convrot::GatedResidual gr{};
+  if (residual)
+    if (int rc = check_residual(residual, gate, gate_stride, rows_per_gate, M, N, &gr)) return rc;
+  return launch_status(convrot::launch_linear_rows(x, dtype, s, a4 != 0, qweight, wscales, bias, M, N, K, out, gr,
+                                                   (hipStream_t)stream),
+                       "convrot_linear_rows");
 }
 
 int convrot_pack_int4(const int8_t* values, int64_t rows, int64_t packed_cols, uint8_t* out, void* stream) {

@@ -248,6 +248,38 @@ __device__ __forceinline__ void nibbles_x16(uint32_t w, uint32_t& lo, uint32_t& 
   hi = w & 0xf0f0f0f0u;
 }
 
+// ---- W4A16 operands
+
+// 8 codes of one CDNA4 weight dword (byte j: feature j low nibble, j+4 high
+// nibble) as 16x-scaled 16-bit floats, natural feature order.
+template <int ADT>
+__device__ __forceinline__ i32x4 expand8(uint32_t w) {
+  uint32_t lo, hi;
+  nibbles_x16(w, lo, hi);
+  float f[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f[j] = (float)(int8_t)(lo >> (8 * j));
+    f[4 + j] = (float)(int8_t)(hi >> (8 * j));
+  }
+  i32x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    r[j] = (int)(ADT == kBF16 ? pack_bf16x2(f[2 * j], f[2 * j + 1]) : pack_f16x2(f[2 * j], f[2 * j + 1]));
+  }
+  return r;
+}
+
+template <int ADT>
+__device__ __forceinline__ f32x4 mfma16(i32x4 a, i32x4 b, f32x4 c) {
+  if constexpr (ADT == kBF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                   0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
+                                                  0, 0);
+}
+
 // ---- direct-to-LDS loads (the DMA GEMM pipelines)
 
 typedef int i32x4_sgpr __attribute__((ext_vector_type(4)));

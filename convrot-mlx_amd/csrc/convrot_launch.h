@@ -28,6 +28,7 @@ enum TuneKey : int {
   kTuneGemmPersist,      // persistent 4-wave W4A4 kernel: 0 never, G > 0 always, on a grid of G workgroups
   kTuneGemmMfma32,       // 1: the 4-wave 256x256 tile on v_mfma_i32_32x32x32_i8
   kTuneFp6Tile,          // FP6 W4A4 tile: bm | bn << 10
+  kTuneRowsCfg,          // few-row linear: weight tiles a workgroup (1, 2, 3, 5), or 16: one tile on 16 waves
   kTuneCount
 };
 int tuning(TuneKey key);
@@ -111,6 +112,14 @@ hipError_t launch_w4a4_gemm_fp6(const uint8_t* act6, const float* xscales, const
 hipError_t launch_w4a4_smallm(const int8_t* act, const float* xscales, const uint8_t* qweight,
                               const float* wscales, const float* bias, int64_t M, int64_t N, int64_t K, void* out,
                               int out_dtype, hipStream_t stream, const GatedResidual& gr = GatedResidual{});
+
+// The ConvRot linear of a few rows in one launch (x to output; linear_rows.hip)
+// and whether it takes a shape: a W4A4 (a4) or W4A16 product of 1 .. 16 rows of
+// at most 32 KB in all, groups of 64 or 256 (log4g 3, 4), K a multiple of 32.
+bool linear_rows_eligible(int64_t M, int64_t K, int dtype, int log4g, bool a4);
+hipError_t launch_linear_rows(const void* x, int dtype, int log4g, bool a4, const uint8_t* qweight,
+                              const float* wscales, const float* bias, int64_t M, int64_t N, int64_t K, void* out,
+                              const GatedResidual& gr, hipStream_t stream);
 
 // Compute units of the current device (cached per device).
 int device_cus();

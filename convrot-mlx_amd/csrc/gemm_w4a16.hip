@@ -25,26 +25,6 @@
 namespace convrot {
 namespace {
 
-// 8 codes of one CDNA4 weight dword (byte j: feature j low nibble, j+4 high
-// nibble) as 16x-scaled 16-bit floats, natural feature order.
-template <int ADT>
-__device__ __forceinline__ i32x4 expand8(uint32_t w) {
-  uint32_t lo, hi;
-  nibbles_x16(w, lo, hi);
-  float f[8];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    f[j] = (float)(int8_t)(lo >> (8 * j));
-    f[4 + j] = (float)(int8_t)(hi >> (8 * j));
-  }
-  i32x4 r;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    r[j] = (int)(ADT == kBF16 ? pack_bf16x2(f[2 * j], f[2 * j + 1]) : pack_f16x2(f[2 * j], f[2 * j + 1]));
-  }
-  return r;
-}
-
 // Activation fragments of one 128-feature block.  Load c gives lane
 // L = 16 u1 + 4 u0 + j the 8 features 32 u1 + 8 j .. +7 of token row
 // 4 u0 + c, so the 16 lanes of each 4-lane quad group read a row's 256
@@ -73,16 +53,6 @@ __device__ __forceinline__ void transpose_quads4(i32x4 (&a)[4], uint8_t* buf, in
 #pragma unroll
   for (int s = 0; s < 4; ++s) a[s] = *(const i32x4*)(buf + (r & 3) * kXposeStride + (16 * q + 4 * (r >> 2) + s) * 16);
   wave_lds_fence();  // the buffer's next writes come after these reads
-}
-
-template <int ADT>
-__device__ __forceinline__ f32x4 mfma16(i32x4 a, i32x4 b, f32x4 c) {
-  if constexpr (ADT == kBF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
-                                                  0, 0);
 }
 
 // Split of K over workgroups (grid.z): workgroup z takes the k-blocks

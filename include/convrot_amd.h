@@ -126,6 +126,24 @@ int convrot_prepare_gelu(const void* head, int64_t head_features, int64_t head_s
                          void* out, float* scales, void* stream);
 
 /*
+ * The ConvRot linear of a few rows in one launch, from x to the output:
+ *   a4 != 0: convrot_prepare(INT8), then convrot_w4a4_gemm (the same bits);
+ *   a4 == 0: convrot_prepare(ROTATE), then convrot_w4a16_gemm (float32 sums in
+ *            an order of its own), both as ConvRotLinear runs them
+ *            (core.py:1270-1313), in x's dtype throughout.
+ * Every workgroup prepares the rows itself while its weights are on their way.
+ * x: dtype [M, K] contiguous, 1 <= M <= 16, M * K elements of at most 32 KB in
+ * all; group_size 64 or 256, K % group_size == 0; a4 == 0: dtype F16 or BF16.
+ * qweight: CDNA4; wscales, bias, residual, gate (NULL: none) as in
+ * convrot_w4a4_gemm_ws; out: dtype [M, N], may be the residual but must not
+ * overlap x (CONVROT_ERR_INVALID).  Other shapes: CONVROT_ERR_UNSUPPORTED.
+ */
+int convrot_linear_rows(const void* x, int dtype, int group_size, int a4, const uint8_t* qweight,
+                        const float* wscales, const float* bias, int64_t M, int64_t N, int64_t K,
+                        const void* residual, const void* gate, int64_t gate_stride, int64_t rows_per_gate, void* out,
+                        void* stream);
+
+/*
  * W4A4 GEMM with fused epilogue:
  *   out[m, n] = out_dtype(((float(sum_k a[m,k] * w[n,k]) * xscales[m]) * wscales[n]) + bias[n])
  * (left to right, no contraction; integer dot exact in int32).
