@@ -18,9 +18,9 @@ LIB_PATH = Path(__file__).resolve().parent / LIB_NAME
 # include/convrot_amd.h
 DTYPE_F32, DTYPE_F16, DTYPE_BF16 = 0, 1, 2
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_LAUNCH = 0, 1, 2, 3
-PREP_PACKED, PREP_INT8, PREP_ROTATE, PREP_FP6, PREP_NO_ROTATE = 0, 1, 2, 3, 0x10
+PREP_PACKED, PREP_INT8, PREP_ROTATE, PREP_FP6, PREP_INT8_BLOCKED, PREP_NO_ROTATE = 0, 1, 2, 3, 4, 0x10
 LAYOUT_NK, LAYOUT_KN, LAYOUT_CDNA4 = 0, 1, 2
-ACT_PACKED, ACT_INT8 = 0, 1
+ACT_PACKED, ACT_INT8, ACT_INT8_BLOCKED = 0, 1, 2
 
 # Every symbol the header declares, with its ctypes signature.
 _vp, _i64, _i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
@@ -50,6 +50,7 @@ SIGNATURES = {
     "convrot_repack_weight": (_i32, [_vp, _i32, _vp, _i32, _i64, _i64, _vp]),
     "convrot_cdna4_bytes": (_i64, [_i64, _i64]),
     "convrot_fp6_bytes": (_i64, [_i64, _i64]),
+    "convrot_w4a4_blocked": (_i32, [_i64, _i64, _i64]),
     "convrot_w4a4_fp6_tile": (_i32, [_i64, _i64, _vp, _vp]),
     "convrot_weight_fp6": (_i32, [_vp, _vp, _i64, _i64, _vp]),
     "convrot_w4a4_gemm_fp6": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i32, _vp]),
@@ -144,7 +145,7 @@ def set_tuning(name: str, value: str | None) -> None:
     gemm_sk_min, gemm_no_dma, gemm_smallm_max, w4a4_smallm_cfg (A/B/C/F), w4a16_cfg
     (A/B/C/D/E/F, S: split K, T), w4a16_tile ("BMxBN"), prep_ni (1/3/4), sk_spin_limit, gemm_persist (0: never;
     G: always, on G workgroups), gemm_mfma32 (0/1), fp6_tile ("BMxBN": 256x256, 256x224, 128x256, 128x192, 128x128),
-    linear_rows_cfg (1/2/3/5/16)."""
+    linear_rows_cfg (1/2/3/5/16), w4a4_midm_cfg (10 * row tiles + weight tiles)."""
     check(load().convrot_set_tuning(name.encode(), None if value is None else str(value).encode()))
 
 

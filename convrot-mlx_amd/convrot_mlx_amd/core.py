@@ -94,6 +94,11 @@ def fp6_shape(rows: int, features: int) -> tuple[int, int, int]:
     return (features // 128, -(-rows // 16), 1536)
 
 
+def _int8_blocked_shape(rows: int, features: int) -> tuple[int, int, int]:
+    """Shape of a [rows, features] activation's int8 codes in CONVROT_PREP_INT8_BLOCKED blocks."""
+    return (-(-features // 128), -(-rows // 16), 2048)
+
+
 def _prep_out(kind: int, rows: int, features: int, like: torch.Tensor) -> torch.Tensor:
     """Output buffer of a preparation mode (FP6 blocks of a ragged last row block are
     only partly written; their padding rows only reach GEMM rows that are never stored)."""
@@ -101,6 +106,8 @@ def _prep_out(kind: int, rows: int, features: int, like: torch.Tensor) -> torch.
         return torch.empty((rows, features // 2), dtype=torch.uint8, device=like.device)
     if kind == nat.PREP_INT8:
         return torch.empty((rows, features), dtype=torch.int8, device=like.device)
+    if kind == nat.PREP_INT8_BLOCKED:
+        return torch.empty(_int8_blocked_shape(rows, features), dtype=torch.int8, device=like.device)
     if kind == nat.PREP_FP6:
         return torch.empty(fp6_shape(rows, features), dtype=torch.uint8, device=like.device)
     return torch.empty((rows, features), dtype=like.dtype, device=like.device)
@@ -579,8 +586,8 @@ def w4a4_status(device=None) -> None:
 
 
 def _w4a4(act: torch.Tensor, act_format: int, k: int, qweight, xscales, wscales, bias, output_dtype, n=None,
-          gr: GatedResidual | None = None):
-    m = act.shape[0]
+          gr: GatedResidual | None = None, m=None):
+    m = m if m is not None else act.shape[0]
     n_layout = _weight_n(qweight, k)
     n = n if n is not None else n_layout
     if k % 32:
@@ -907,6 +914,11 @@ def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, 
     return out
 
 
+def _blocked_codes(m: int, n: int, k: int) -> bool:
+    """Whether a W4A4 product on INT8 operands runs on blocked codes in ConvRotLinear."""
+    return 4 < m < 256 and bool(nat.load().convrot_w4a4_blocked(m, n, k))
+
+
 # Reference names (the reference's Metal/MPP entry points) -> the gfx950 kernels.
 metal_fused_prepare_convrot_activation = hip_fused_prepare_convrot_activation
 metal_fused_prepare_convrot_activation_i8 = hip_fused_prepare_convrot_activation_i8
@@ -1065,6 +1077,10 @@ class ConvRotLinear(nn.Module):
             act6, xscales = prep(nat.PREP_FP6)
             out = _w4a4_fp6(act6, w6, xscales, self.scales, self.bias, dtype, rows, self.out_features,
                             self.in_features, gr)
+        elif self.a4 and _blocked_codes(rows, self.out_features, self.in_features):
+            qact, xscales = prep(nat.PREP_INT8_BLOCKED)
+            out = _w4a4(qact, nat.ACT_INT8_BLOCKED, self.in_features, w, xscales, self.scales, self.bias, dtype,
+                        self.out_features, gr, rows)
         elif self.a4:
             qact, xscales = prep(nat.PREP_INT8)
             out = _w4a4(qact, nat.ACT_INT8, self.in_features, w, xscales, self.scales, self.bias, dtype,

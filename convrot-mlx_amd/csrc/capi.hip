@@ -97,7 +97,8 @@ int convrot_set_tuning(const char* name, const char* value) {
                 {"w4a16_cfg", kTuneW4a16Cfg},         {"w4a16_tile", kTuneW4a16Tile},
                 {"prep_ni", kTunePrepNi},             {"sk_spin_limit", kTuneSkSpinLimit},
                 {"gemm_persist", kTuneGemmPersist},   {"gemm_mfma32", kTuneGemmMfma32},
-                {"fp6_tile", kTuneFp6Tile},           {"linear_rows_cfg", kTuneRowsCfg}};
+                {"fp6_tile", kTuneFp6Tile},           {"linear_rows_cfg", kTuneRowsCfg},
+                {"w4a4_midm_cfg", kTuneMidmCfg}};
   int key = -1;
   for (const auto& n : kNames)
     if (strcmp(n.name, name) == 0) key = n.key;
@@ -135,6 +136,10 @@ int convrot_set_tuning(const char* name, const char* value) {
         v = atoi(value);
         good = v == 1 || v == 2 || v == 3 || v == 5 || v == 16;
         break;
+      case kTuneMidmCfg:
+        v = atoi(value);
+        good = midm_split_known(v);
+        break;
       default: {
         char* end = nullptr;
         const long long n = strtoll(value, &end, 10);
@@ -160,6 +165,8 @@ int64_t convrot_fp6_bytes(int64_t R, int64_t K) {
   return (K / 128) * ((R + 15) / 16) * 1536;
 }
 
+int convrot_w4a4_blocked(int64_t M, int64_t N, int64_t K) { return convrot::midm_preferred(M, N, K) ? 1 : 0; }
+
 int convrot_w4a4_fp6_tile(int64_t M, int64_t N, int* bm, int* bn) {
   if (M <= 0 || N <= 0 || !bm || !bn)
     return fail(CONVROT_ERR_INVALID, "FP6 tile query needs M, N > 0 and two result pointers");
@@ -172,7 +179,7 @@ int convrot_prepare(const void* x, int dtype, int64_t rows, int64_t features, in
   const bool no_rotate = (mode & CONVROT_PREP_NO_ROTATE) != 0;
   const int kind = mode & ~CONVROT_PREP_NO_ROTATE;
   if (kind != CONVROT_PREP_PACKED && kind != CONVROT_PREP_INT8 && kind != CONVROT_PREP_ROTATE &&
-      kind != CONVROT_PREP_FP6)
+      kind != CONVROT_PREP_FP6 && kind != CONVROT_PREP_INT8_BLOCKED)
     return fail(CONVROT_ERR_INVALID, "unknown ConvRot preparation mode %d", mode);
   if (kind == CONVROT_PREP_FP6 && features % 128)
     return fail(CONVROT_ERR_UNSUPPORTED, "FP6 preparation requires features divisible by 128, got %lld",
@@ -212,7 +219,7 @@ int convrot_prepare_modulated(const void* x, int dtype, int64_t rows, int64_t fe
   if (mode & CONVROT_PREP_NO_ROTATE)
     return fail(CONVROT_ERR_INVALID, "the modulated producer always rotates (no CONVROT_PREP_NO_ROTATE)");
   if (mode != CONVROT_PREP_PACKED && mode != CONVROT_PREP_INT8 && mode != CONVROT_PREP_ROTATE &&
-      mode != CONVROT_PREP_FP6)
+      mode != CONVROT_PREP_FP6 && mode != CONVROT_PREP_INT8_BLOCKED)
     return fail(CONVROT_ERR_INVALID, "unknown ConvRot preparation mode %d", mode);
   if (!valid_dtype(dtype)) return fail(CONVROT_ERR_INVALID, "unsupported activation dtype code %d", dtype);
   if (rows < 0 || features <= 0) return fail(CONVROT_ERR_INVALID, "invalid shape (%lld, %lld)", (long long)rows, (long long)features);
@@ -250,7 +257,7 @@ int convrot_prepare_gelu(const void* head, int64_t head_features, int64_t head_s
   if (mode & CONVROT_PREP_NO_ROTATE)
     return fail(CONVROT_ERR_INVALID, "the GELU producer always rotates (no CONVROT_PREP_NO_ROTATE)");
   if (mode != CONVROT_PREP_PACKED && mode != CONVROT_PREP_INT8 && mode != CONVROT_PREP_ROTATE &&
-      mode != CONVROT_PREP_FP6)
+      mode != CONVROT_PREP_FP6 && mode != CONVROT_PREP_INT8_BLOCKED)
     return fail(CONVROT_ERR_INVALID, "unknown ConvRot preparation mode %d", mode);
   if (!valid_dtype(dtype)) return fail(CONVROT_ERR_INVALID, "unsupported activation dtype code %d", dtype);
   if (rows < 0 || head_features < 0 || x_features <= 0)
@@ -293,7 +300,7 @@ namespace {
 // launch may proceed (M == 0 or N == 0 included).
 int check_w4a4(const void* act, int act_format, const float* xscales, const uint8_t* qweight,
                const float* wscales, int64_t M, int64_t N, int64_t K, void* out, int out_dtype) {
-  if (act_format != CONVROT_ACT_PACKED && act_format != CONVROT_ACT_INT8)
+  if (act_format != CONVROT_ACT_PACKED && act_format != CONVROT_ACT_INT8 && act_format != CONVROT_ACT_INT8_BLOCKED)
     return fail(CONVROT_ERR_INVALID, "unknown activation format %d", act_format);
   if (!valid_dtype(out_dtype)) return fail(CONVROT_ERR_INVALID, "unsupported output dtype code %d", out_dtype);
   if (M < 0 || N < 0 || K <= 0) return fail(CONVROT_ERR_INVALID, "invalid GEMM shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
@@ -301,6 +308,9 @@ int check_w4a4(const void* act, int act_format, const float* xscales, const uint
   if (K > kMaxFeatures)
     return fail(CONVROT_ERR_UNSUPPORTED, "W4A4 GEMM supports K up to %lld, got %lld", (long long)kMaxFeatures, (long long)K);
   if (M > 0x7fffffff || N > 0x7fffffff) return fail(CONVROT_ERR_UNSUPPORTED, "GEMM dimension too large");
+  if (act_format == CONVROT_ACT_INT8_BLOCKED && ((K + 127) / 128) * ((M + 15) / 16) * 2048 >= kMaxWeightBytes)
+    return fail(CONVROT_ERR_UNSUPPORTED, "blocked activations are limited to 2 GiB (M=%lld K=%lld)", (long long)M,
+                (long long)K);
   if (packed_weight_bytes(N, K) >= kMaxWeightBytes)
     return fail(CONVROT_ERR_UNSUPPORTED, "W4A4 GEMM packed weights are limited to 2 GiB (N=%lld K=%lld)", (long long)N,
                 (long long)K);

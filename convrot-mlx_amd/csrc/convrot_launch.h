@@ -29,6 +29,7 @@ enum TuneKey : int {
   kTuneGemmMfma32,       // 1: the 4-wave 256x256 tile on v_mfma_i32_32x32x32_i8
   kTuneFp6Tile,          // FP6 W4A4 tile: bm | bn << 10
   kTuneRowsCfg,          // few-row linear: weight tiles a workgroup (1, 2, 3, 5), or 16: one tile on 16 waves
+  kTuneMidmCfg,          // W4A4 kernel of blocked codes: 10 * row tiles + weight tiles of a workgroup
   kTuneCount
 };
 int tuning(TuneKey key);
@@ -107,11 +108,24 @@ hipError_t launch_w4a4_gemm_fp6(const uint8_t* act6, const float* xscales, const
                                 const float* bias, int64_t M, int64_t N, int64_t K, void* out, int out_dtype,
                                 hipStream_t stream, const GatedResidual& gr, bool compact_weights = false);
 
+// The few-row W4A4 kernel takes up to 64 rows while the int4 weight is at most
+// ~20 MB (N * K elements), else 32.
+constexpr int64_t kSmallMWideElems = 40000000;
+
 // Few-row W4A4 kernel (int8 activation codes only); launch_w4a4_gemm routes
 // small M here.
 hipError_t launch_w4a4_smallm(const int8_t* act, const float* xscales, const uint8_t* qweight,
                               const float* wscales, const float* bias, int64_t M, int64_t N, int64_t K, void* out,
                               int out_dtype, hipStream_t stream, const GatedResidual& gr = GatedResidual{});
+
+// W4A4 kernel for tens to a few hundred rows (blocked int8 codes, eight waves
+// splitting K): the row and weight tiles of a workgroup its plan picks.
+void midm_plan(int64_t M, int64_t N, int64_t K, int* fm, int* nb);
+bool midm_preferred(int64_t M, int64_t N, int64_t K);  // over the kernels of row-major codes
+bool midm_split_known(int cfg);                        // 10 * row tiles + weight tiles
+hipError_t launch_w4a4_midm(const uint8_t* act, const float* xscales, const uint8_t* qweight, const float* wscales,
+                            const float* bias, int64_t M, int64_t N, int64_t K, void* out, int out_dtype,
+                            hipStream_t stream, const GatedResidual& gr);
 
 // The ConvRot linear of a few rows in one launch (x to output; linear_rows.hip)
 // and whether it takes a shape: a W4A4 (a4) or W4A16 product of 1 .. 16 rows of

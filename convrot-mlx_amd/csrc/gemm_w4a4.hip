@@ -2422,7 +2422,6 @@ hipError_t launch_odt(int odt, const void* act, const float* xs, const uint8_t* 
 
 constexpr int64_t kSmallMMax = 32;
 constexpr int64_t kSmallMMaxWide = 64;
-constexpr int64_t kSmallMWideElems = 40000000;  // N * K, i.e. 20 MB of int4 weights
 
 namespace {
 
@@ -2443,6 +2442,8 @@ hipError_t launch_w4a4_gemm(const void* act, int act_format, const float* xscale
                             void* out, int out_dtype, hipStream_t stream, const GatedResidual& gr,
                             WorkspaceSource src) {
   if (M == 0 || N == 0) return hipSuccess;
+  if (act_format == CONVROT_ACT_INT8_BLOCKED)
+    return launch_w4a4_midm((const uint8_t*)act, xscales, qweight, wscales, bias, M, N, K, out, out_dtype, stream, gr);
   if (act_format == CONVROT_ACT_PACKED)
     return launch_odt<true>(out_dtype, act, xscales, qweight, wscales, bias, M, N, K, out, gr, src, stream);
   if (M <= smallm_limit(N, K))
@@ -2464,7 +2465,7 @@ bool w4a4_tile_known(int bm, int bn, int wm, int wn, int stages) {
 }
 
 size_t w4a4_plan_workspace_bytes(int act_format, int64_t M, int64_t N, int64_t K) {
-  if (M == 0 || N == 0 || act_format == CONVROT_ACT_PACKED || M <= smallm_limit(N, K)) return 0;
+  if (M == 0 || N == 0 || act_format != CONVROT_ACT_INT8 || M <= smallm_limit(N, K)) return 0;
   const bool dma = tuning(kTuneGemmNoDma) != 1;
   const Plan plan = choose_plan(M, N, K, dma, dma ? kSkWorkspaceBytes : 0);
   return plan.sk ? sk_bytes(plan.t, plan.grid) : 0;

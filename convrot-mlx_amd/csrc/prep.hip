@@ -183,8 +183,8 @@ __global__ __launch_bounds__(1024) void prep_kernel(const void* __restrict__ x, 
   const int wave = threadIdx.x >> 6;
   const int nwaves = blockDim.x >> 6;
   int64_t row = blockIdx.x;
-  if constexpr (MODE == CONVROT_PREP_FP6) {
-    // Workgroups go round-robin to the 8 XCDs.  The 16 rows of an FP6 block
+  if constexpr (MODE == CONVROT_PREP_FP6 || MODE == CONVROT_PREP_INT8_BLOCKED) {
+    // Workgroups go round-robin to the 8 XCDs.  The 16 rows of a block
     // share its cache lines, so each XCD takes runs of consecutive rows (a
     // multiple of 16 each) and its L2 merges the rows' pieces of a line.
     const int64_t run = ((int64_t)gridDim.x / (8 * 16)) * 16;
@@ -409,7 +409,14 @@ __global__ __launch_bounds__(1024) void prep_kernel(const void* __restrict__ x, 
     for (int run = 0; run < 4; ++run) {
       const int64_t f = gbase + run_index<(S >= 3 ? S : 3), PHF>(p, run);
       const float* vr = &v[4 * run];
-      if constexpr (MODE == CONVROT_PREP_INT8) {
+      if constexpr (MODE == CONVROT_PREP_INT8_BLOCKED) {
+        // the blocks the mid-size W4A4 GEMM's MFMA reads: 16 rows x 128 features, 1 KB for each 16-feature half
+        const int fr = (int)(f - row * K);
+        const int64_t mblocks = ((int64_t)gridDim.x + 15) >> 4;
+        uint8_t* blk = (uint8_t*)out + ((int64_t)(fr >> 7) * mblocks + (row >> 4)) * 2048;
+        *(uint32_t*)(blk + (fr & 16) * 64 + (((fr >> 5) & 3) * 16 + (int)(row & 15)) * 16 + (fr & 15)) =
+            gather_bytes(q[4 * run], q[4 * run + 1], q[4 * run + 2], q[4 * run + 3]);
+      } else if constexpr (MODE == CONVROT_PREP_INT8) {
         ((uint32_t*)out)[f >> 2] = gather_bytes(q[4 * run], q[4 * run + 1], q[4 * run + 2], q[4 * run + 3]);
       } else if constexpr (MODE == CONVROT_PREP_PACKED) {
         ((uint16_t*)out)[f >> 2] =
@@ -453,6 +460,8 @@ hipError_t launch_prep_mode(int mode, const void* x, void* out, float* scales, i
       return launch_prep_t<DT, S, NI, CONVROT_PREP_PACKED>(x, out, scales, rows, K, waves, mod, stream);
     case CONVROT_PREP_FP6:
       return launch_prep_t<DT, S, NI, CONVROT_PREP_FP6>(x, out, scales, rows, K, waves, mod, stream);
+    case CONVROT_PREP_INT8_BLOCKED:
+      return launch_prep_t<DT, S, NI, CONVROT_PREP_INT8_BLOCKED>(x, out, scales, rows, K, waves, mod, stream);
     case CONVROT_PREP_INT8:
       return launch_prep_t<DT, S, NI, CONVROT_PREP_INT8>(x, out, scales, rows, K, waves, mod, stream);
     default: return launch_prep_t<DT, S, NI, CONVROT_PREP_ROTATE>(x, out, scales, rows, K, waves, mod, stream);

@@ -57,6 +57,9 @@ extern "C" {
 #define CONVROT_PREP_ROTATE 2 /* out: dtype [rows, features] rotated values (scales unused) */
 #define CONVROT_PREP_FP6 3    /* out: FP6 operand blocks of the A4 codes, + scales; features % 128 == 0
                                * (layout: convrot_w4a4_gemm_fp6; convrot_fp6_bytes(rows, features)) */
+#define CONVROT_PREP_INT8_BLOCKED 4 /* out: int8 A4 codes in [ceil(features/128)][ceil(rows/16)][2048] blocks, + scales:
+                               * feature f = 32 q + 16 s + b (q 0..3, s 0..1, b 0..15) of the block's row r at
+                               * byte 1024 s + 16 (16 q + r) + b; rows and features past the end are not written */
 /* OR-able flag: skip the rotation (quantize_signed_int4_rowwise semantics) */
 #define CONVROT_PREP_NO_ROTATE 0x10
 
@@ -68,6 +71,7 @@ extern "C" {
 /* activation operand formats for convrot_w4a4_gemm */
 #define CONVROT_ACT_PACKED 0 /* uint8 [M, K/2] packed A4 (core.py:1061 mpp_w4a4_matmul) */
 #define CONVROT_ACT_INT8 1   /* int8  [M, K]              (core.py:1088 mpp_w4a4_int8_matmul) */
+#define CONVROT_ACT_INT8_BLOCKED 2 /* the blocks of CONVROT_PREP_INT8_BLOCKED (below 2 GiB) */
 
 /*
  * Fused activation preparation: normalized regular-Hadamard rotation of each
@@ -161,6 +165,11 @@ int convrot_w4a4_gemm(const void* act, int act_format, const float* xscales,
                       const uint8_t* qweight, const float* wscales, const float* bias,
                       int64_t M, int64_t N, int64_t K, void* out, int out_dtype,
                       void* stream);
+
+/* 1 where convrot_w4a4_gemm runs an M x N x K product faster on blocked codes
+ * (CONVROT_PREP_INT8_BLOCKED, CONVROT_ACT_INT8_BLOCKED) than on row-major ones:
+ * tens to a few hundred rows.  The outputs are the same bits. */
+int convrot_w4a4_blocked(int64_t M, int64_t N, int64_t K);
 
 /*
  * convrot_w4a4_gemm followed, inside the same kernel, by a gated residual:
