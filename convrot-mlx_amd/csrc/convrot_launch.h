@@ -44,7 +44,7 @@ bool w4a16_tile_known(int bm, int bn);
 // The FP6 W4A4 tile the plan (and the fp6_tile override) picks for M x N.
 void fp6_plan_tile(int64_t M, int64_t N, int* bm, int* bn);
 
-bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out);
+bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out, bool packed);
 
 hipError_t launch_prep(const void* x, int dtype, int64_t rows, int64_t K, int log4g, int mode, void* out,
                        float* scales, hipStream_t stream);

@@ -110,25 +110,36 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
 //   y = (0.5 * x) * (1 + tanh(u))
 // with exp(z) = 2^n e^r, n = rint(z log2 e), r = z - n ln2 by two fmas
 // (Cody-Waite), e^r by its degree-7 Taylor polynomial (Horner, fma).
+//
+// Cheaper forms of the same values:
+//  * rint by adding and subtracting 1.5 * 2^23 (|z log2 e| < 2^7), which leaves
+//    n in the low bits of the sum: 2^n p is an integer add to p's exponent
+//    (p in [0.7, 1.42], n <= 127: no overflow, no denormal);
+//  * 2 / s as the reciprocal of s / 2 (exact halving), the reciprocal by one
+//    Newton step from v_rcp_f32 (correctly rounded for every s / 2 in
+//    [1, 2^126): checked over all significands, tests/test_gpu_prep16.py).
+// 35 VALU operations with a conversion and a division in them became 29.
 __device__ __forceinline__ float gelu_tanh32(float x) {
   const float x3 = (x * x) * x;
   const float u = 0x1.988454p-1f * __builtin_fmaf(0x1.6e4e26p-5f, x3, x);
   const float z = fabsf(u) + fabsf(u);
-  float q = 0.0f;
-  if (z <= 88.0f) {
-    const float n = rintf(z * 0x1.715476p+0f);
-    float r = __builtin_fmaf(-n, 0x1.62e4p-1f, z);
-    r = __builtin_fmaf(-n, 0x1.7f7d1cp-20f, r);
-    float p = 0x1.a01a02p-13f;
-    p = __builtin_fmaf(p, r, 0x1.6c16c2p-10f);
-    p = __builtin_fmaf(p, r, 0x1.111112p-7f);
-    p = __builtin_fmaf(p, r, 0x1.555556p-5f);
-    p = __builtin_fmaf(p, r, 0x1.555556p-3f);
-    p = __builtin_fmaf(p, r, 0x1p-1f);
-    p = __builtin_fmaf(p, r, 1.0f);
-    p = __builtin_fmaf(p, r, 1.0f);
-    q = 2.0f / (ldexpf(p, (int)n) + 1.0f);
-  }
+  const float t = z * 0x1.715476p+0f + 12582912.0f;
+  const float n = t - 12582912.0f;
+  float r = __builtin_fmaf(-n, 0x1.62e4p-1f, z);
+  r = __builtin_fmaf(-n, 0x1.7f7d1cp-20f, r);
+  float p = 0x1.a01a02p-13f;
+  p = __builtin_fmaf(p, r, 0x1.6c16c2p-10f);
+  p = __builtin_fmaf(p, r, 0x1.111112p-7f);
+  p = __builtin_fmaf(p, r, 0x1.555556p-5f);
+  p = __builtin_fmaf(p, r, 0x1.555556p-3f);
+  p = __builtin_fmaf(p, r, 0x1p-1f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  const float e = __uint_as_float(__float_as_uint(p) + (__float_as_uint(t) << 23));
+  const float d = 0.5f * (e + 1.0f);
+  const float y = __builtin_amdgcn_rcpf(d);
+  const float qr = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+  const float q = z <= 88.0f ? qr : 0.0f;
   const float onept = u >= 0.0f ? 2.0f - q : q;
   return (0.5f * x) * onept;
 }
@@ -430,6 +441,536 @@ __global__ __launch_bounds__(1024) void prep_kernel(const void* __restrict__ x, 
   }
 }
 
+// ---- 16-bit activations, two to a register
+//
+// The butterfly's cost is its rounding: with one value a register every add is
+// a v_add_f32 and a conversion that rounds a single value (20 operations a
+// radix-4, 5 a value and stage; MI355X issues a conversion every 1.9 ns a
+// SIMD, an add every 1.3).  Here the values stay packed in x's type:
+//  * float16: v_pk_add_f16, whose sum is the float32 sum rounded (24 >= 2 * 11
+//    + 2 bits: rounding twice changes nothing), 1.25 operations a value and stage;
+//  * bfloat16, which has no packed add: v_mfma_f32_4x4x4_16b_bf16 as one.  Its B
+//    operand is the lane's own four values (two registers) and its A operand a
+//    constant 4 x 4 matrix of 0, 1 and -1, so a lane's four results are sums and
+//    differences of its values, which one conversion packs two at a time.  Every
+//    such sum of two finite bf16 values, rounded to bf16, is the float32 sum
+//    rounded (all 2^32 pairs and the denormals checked on the GPU, whatever the
+//    other two values are: their products are zeros): where the exponents are
+//    within 16 the sum is exact in 24 bits, beyond that both round to the larger.
+//    1.25 conversions a value and stage are left to the vector unit; the matrix
+//    unit's 0.9 instructions run beside them.
+// An infinity or NaN would reach the lane's other sums as 0 * inf, so a wave
+// that ends with one (or with an overflow) rotates its share again in float32;
+// only signs of zeros differ, which no code keeps (so ROTATE outputs of bf16
+// stay with the kernel above); float16 rows take the same way (only the sign of
+// a NaN may differ from prep_kernel's there).
+//
+// FP6 output, prep_kernel -> this kernel (back-to-back launches over cold
+// buffers, us): bf16 G = 256 4608 x 3072 16.6 -> 13.8, 4608 x 15360 59.5 -> 51.7
+// (3.8 TB/s), 8800 x 16384 112 -> 101-104, GELU 8800 x 16384 215 -> 172; float16
+// 10017 x 2688 31.3 -> 23.5, 8800 x 16384 150 -> 103; packed output bf16
+// 12288 x 3072 35.1 -> 26.5.  What is left above the bytes (8800 x 16384: 397 MB,
+// 78 us at a copy's 5.1 TB/s) is the vector work, still 60 % of that time, where
+// it does not overlap the loads, and the FP6 slots' 16-byte stores.
+// Registers for 5, 6 and 8 waves a SIMD at 4, 3 and 1 iterations: left alone the
+// compiler takes 4 waves' worth (4608 x 3072: 15.2 us).
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// A lane's rows of the constant matrices (row lane % 4 of each 4 x 4), applied
+// to B = (x0, x1, y0, y1):
+//   sum   x0 + y0, x1 + y1, x0 - y0, x1 - y1
+//   id    x0, x1, y0, y1
+//   minus -y0, -y1, y0, y1       plus  y0, y1, y0, y1
+// and on a run (a, b, c, d) of digit 0:
+//   t     t1 = a + b, t2 = a - b (0, 0)       last  -d, d, d, d
+//   u     on (t1, t2, c, d): u0 = t1 + c, u1 = t1 - c, u2 = t2 + c, u3 = c - t2
+// id with the +-d of minus, plus or last as the accumulator adds a stage's last
+// term to all four sums at once.
+struct Matrices {
+  uint2 sum, id, minus, plus, t, last, u;
+};
+
+__device__ __forceinline__ Matrices matrices(int lane) {
+  const uint32_t P0 = 0x3f80u, N0 = 0xbf80u, P1 = P0 << 16, N1 = N0 << 16;  // +-1 in the low / high half
+  const int i = lane & 3;
+  const auto row = [i](uint32_t a, uint32_t b, uint32_t c, uint32_t d) { return i == 0 ? a : i == 1 ? b : i == 2 ? c : d; };
+  Matrices m;
+  m.sum = make_uint2(row(P0, P1, P0, P1), row(P0, P1, N0, N1));
+  m.id = make_uint2(row(P0, P1, 0u, 0u), row(0u, 0u, P0, P1));
+  m.minus = make_uint2(0u, row(N0, N1, P0, P1));
+  m.plus = make_uint2(0u, row(P0, P1, P0, P1));
+  m.t = make_uint2(row(P0 | P1, P0 | N1, 0u, 0u), 0u);
+  m.last = make_uint2(0u, row(N1, P1, P1, P1));
+  m.u = make_uint2(row(P0, P0, P1, N1), row(P0, N0, P0, P0));
+  return m;
+}
+
+__device__ __forceinline__ f32x4 mfma4(uint2 a, uint32_t x, uint32_t y, f32x4 c = (f32x4){0.f, 0.f, 0.f, 0.f}) {
+  const uint2 b = make_uint2(x, y);
+  return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f16x2 as_f16(uint32_t w) { return __builtin_bit_cast(f16x2, w); }
+__device__ __forceinline__ uint32_t as_u32(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+
+template <int DT>
+__device__ __forceinline__ float pk_lo(uint32_t w) {
+  if constexpr (DT == kBF16) return bf16_lo(w);
+  else return (float)as_f16(w).x;
+}
+template <int DT>
+__device__ __forceinline__ float pk_hi(uint32_t w) {
+  if constexpr (DT == kBF16) return bf16_hi(w);
+  else return (float)as_f16(w).y;
+}
+template <int DT>
+__device__ __forceinline__ uint32_t pk_make(float lo, float hi) {
+  if constexpr (DT == kBF16) return pack_bf16x2(lo, hi);
+  else return pack_f16x2(lo, hi);
+}
+
+// One radix-4 along digit 0 on a packed run (a, b), (c, d); in radix4's order.
+// EXACT: by radix4 itself, for values that may not be finite.
+template <int DT, bool EXACT>
+__device__ __forceinline__ void pk_stage_run(const Matrices& m, uint32_t& x, uint32_t& y) {
+  if constexpr (EXACT) {
+    float a = pk_lo<DT>(x), b = pk_hi<DT>(x), c = pk_lo<DT>(y), d = pk_hi<DT>(y);
+    asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));  // float32 adds (a v_fma_mix negates a NaN)
+    radix4<DT>(a, b, c, d);
+    x = pk_make<DT>(a, b);
+    y = pk_make<DT>(c, d);
+  } else if constexpr (DT == kBF16) {
+    const f32x4 d = mfma4(m.last, x, y), t = mfma4(m.t, x, y);
+    const f32x4 u = mfma4(m.u, pack_bf16x2(t[0], t[1]), y);
+    const f32x4 o = mfma4(m.id, pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), d);
+    x = pack_bf16x2(o[0], o[1]);
+    y = pack_bf16x2(o[2], o[3]);
+  } else {
+    const f16x2 ab = as_f16(x), cd = as_f16(y);
+    const f16x2 t = ab.xx + (f16x2){ab.y, -ab.y};
+    const f16x2 u01 = t.xx + (f16x2){cd.x, -cd.x}, u23 = (f16x2){t.y, -t.y} + cd.xx;
+    x = as_u32(u01 + (f16x2){-cd.y, cd.y});
+    y = as_u32(u23 + cd.yy);
+  }
+}
+
+// Two radix-4s side by side, the digit across four registers.
+template <int DT, bool EXACT>
+__device__ __forceinline__ void pk_stage_regs(const Matrices& m, uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+  if constexpr (EXACT) {
+    float l[4] = {pk_lo<DT>(a), pk_lo<DT>(b), pk_lo<DT>(c), pk_lo<DT>(d)};
+    float h[4] = {pk_hi<DT>(a), pk_hi<DT>(b), pk_hi<DT>(c), pk_hi<DT>(d)};
+    asm volatile("" : "+v"(l[0]), "+v"(l[1]), "+v"(l[2]), "+v"(l[3]), "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]));
+    radix4<DT>(l[0], l[1], l[2], l[3]);
+    radix4<DT>(h[0], h[1], h[2], h[3]);
+    a = pk_make<DT>(l[0], h[0]);
+    b = pk_make<DT>(l[1], h[1]);
+    c = pk_make<DT>(l[2], h[2]);
+    d = pk_make<DT>(l[3], h[3]);
+  } else if constexpr (DT == kBF16) {
+    const f32x4 t = mfma4(m.sum, a, b), dm = mfma4(m.minus, c, d), dp = mfma4(m.plus, c, d);
+    const f32x4 u01 = mfma4(m.sum, pack_bf16x2(t[0], t[1]), c), u23 = mfma4(m.sum, c, pack_bf16x2(t[2], t[3]));
+    const f32x4 o01 = mfma4(m.id, pack_bf16x2(u01[0], u01[1]), pack_bf16x2(u01[2], u01[3]), dm);
+    const f32x4 o23 = mfma4(m.id, pack_bf16x2(u23[0], u23[1]), pack_bf16x2(u23[2], u23[3]), dp);
+    a = pack_bf16x2(o01[0], o01[1]);
+    b = pack_bf16x2(o01[2], o01[3]);
+    c = pack_bf16x2(o23[0], o23[1]);
+    d = pack_bf16x2(o23[2], o23[3]);
+  } else {
+    const f16x2 va = as_f16(a), vb = as_f16(b), vc = as_f16(c), vd = as_f16(d);
+    const f16x2 t1 = va + vb, t2 = va - vb;
+    a = as_u32((t1 + vc) - vd);
+    b = as_u32((t1 - vc) + vd);
+    c = as_u32((t2 + vc) + vd);
+    d = as_u32((vc - t2) + vd);
+  }
+}
+
+// A run of four packed features in the wave's LDS: its two dwords lie in two
+// planes of kPlane dwords, one dword of padding after every four runs
+// (conflict-free but for phase 3's two-way).  In planes a lane reads the same
+// dword of two runs with one ds_read2_b32, into the register pair that the
+// stage's MFMA takes; whole runs (8 bytes) would leave the pairs to v_movs.
+constexpr int kPlane = 324;  // past a ds_read2's offsets and no multiple of 64: the planes are not paired
+constexpr int kPkRegion = 2 * kPlane;  // dwords of a wave's LDS (the FP6 output's transpose takes 512)
+__device__ __forceinline__ int pk_off(int i) { return (i >> 2) + (i >> 4); }
+
+template <int DT, int S, int PH, bool EXACT>
+__device__ __forceinline__ void pk_exchange_and_stage(const Matrices& m, uint32_t (&h)[8], uint32_t* region, int p) {
+#pragma unroll
+  for (int run = 0; run < 4; ++run) {
+    uint32_t* at = region + pk_off(run_index<S, PH - 1>(p, run));
+    at[0] = h[2 * run];
+    at[kPlane] = h[2 * run + 1];
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int run = 0; run < 4; ++run) {
+    const uint32_t* at = region + pk_off(run_index<S, PH>(p, run));
+    h[2 * run] = at[0];
+    h[2 * run + 1] = at[kPlane];
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) pk_stage_regs<DT, EXACT>(m, h[i], h[2 + i], h[4 + i], h[6 + i]);
+}
+
+// rotate16 on packed values (h[2 * run], h[2 * run + 1]: a run's four features).
+template <int DT, int S, bool EXACT = false>
+__device__ __forceinline__ void pk_rotate16(const Matrices& m, uint32_t (&h)[8], uint32_t* region, int p) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) pk_stage_run<DT, EXACT>(m, h[2 * r], h[2 * r + 1]);
+  if constexpr (S >= 2) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) pk_stage_regs<DT, EXACT>(m, h[i], h[2 + i], h[4 + i], h[6 + i]);
+  }
+  if constexpr (S >= 3) pk_exchange_and_stage<DT, S, 2, EXACT>(m, h, region, p);
+  if constexpr (S >= 4) pk_exchange_and_stage<DT, S, 3, EXACT>(m, h, region, p);
+  if constexpr (S >= 5) pk_exchange_and_stage<DT, S, 4, EXACT>(m, h, region, p);
+}
+
+// 16 consecutive 16-bit elements at byte `off` of a row (past its end: zeros).
+__device__ __forceinline__ void pk_load16(__amdgpu_buffer_rsrc_t row, uint32_t off, uint32_t (&h)[8]) {
+  const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(row, (int)off, 0, 0);
+  const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(row, (int)(off + 16), 0, 0);
+  h[0] = a.x, h[1] = a.y, h[2] = a.z, h[3] = a.w, h[4] = b.x, h[5] = b.y, h[6] = b.z, h[7] = b.w;
+}
+
+// Largest magnitude of 16 packed values, folded into the halves of `m` as bit
+// patterns (they order like the magnitudes, infinity and NaN on top).
+__device__ __forceinline__ uint32_t pk_absmax(uint32_t m, const uint32_t (&h)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const u16x2 v = __builtin_bit_cast(u16x2, h[i] & 0x7fff7fffu);
+    m = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m), v));
+  }
+  return m;
+}
+
+// The float16 ratio of a finite value to a finite scale from inv = 1 / scale
+// (0 for a zero scale): one correction step, whose float32 quotient rounds to
+// the float16 the true division's rounds to (checked over every pair of
+// significands, tests/test_prep16.py).
+__device__ __forceinline__ float f16_quotient(float v, float scale, float inv) {
+  const float q = v * inv;
+  return __builtin_fmaf(__builtin_fmaf(-q, scale, v), inv, q);
+}
+
+// Two packed ratios clamped to [-7, 7] (a float16 scale may be a denormal far
+// below absmax / 7), with +0 for the codes that are zero.
+__device__ __forceinline__ uint32_t f16_clamp_sign_fix(uint32_t w) {
+  const f16x2 seven = {(_Float16)7.0f, (_Float16)7.0f};
+  const uint32_t h = as_u32(__builtin_elementwise_max(__builtin_elementwise_min(as_f16(w), seven), -seven));
+  const u16x2 s = __builtin_bit_cast(u16x2, h) + (u16x2){0x47ff, 0x47ff};  // bit 15: negative, at most 0.5
+  return h & ~(__builtin_bit_cast(uint32_t, s) & 0x80008000u);
+}
+
+typedef _Float16 f16x32 __attribute__((ext_vector_type(32)));
+
+template <int DT>
+__device__ __forceinline__ void pk_fp6_fields16(const uint32_t (&hp)[8], uint32_t& d0, uint32_t& d1, uint32_t& d2) {
+  if constexpr (DT == kBF16) {
+    fp6_fields16(hp, d0, d1, d2);
+  } else {
+    const u32x16 in = {hp[0], hp[1], hp[2], hp[3], hp[4], hp[5], hp[6], hp[7], 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+    const i32x6 f = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(__builtin_bit_cast(f16x32, in), 8.0f);
+    d0 = (uint32_t)f[0];
+    d1 = (uint32_t)f[1];
+    d2 = (uint32_t)f[2];
+  }
+}
+
+// prep_kernel for 16-bit x with S >= 1 (bf16: not ROTATE), the same work split
+// and the same bits.
+template <int DT, int S, int NI, int MODE, int PRO>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(PRO == kProModulate ? 4 : NI == 4 || S == 5 ? 5 : NI == 3 ? 6 : 8)))
+void prep16_kernel(const void* __restrict__ x, void* __restrict__ out,
+                                                       float* __restrict__ scales, int K, ProducerArgs pa) {
+  static_assert(S >= 1 && (DT == kF16 || (DT == kBF16 && MODE != CONVROT_PREP_ROTATE)), "see above");
+  constexpr bool PRE = PRO == kProModulate;
+  extern __shared__ uint32_t lds16[];
+  uint32_t* const lds = lds16;
+  __shared__ float wave_max[kMaxWaves];
+  __shared__ double block_moments[PRE ? kMaxBlocks : 1][2];
+
+  constexpr int G = 1 << (2 * S);
+  constexpr int LG = (S >= 3) ? (G / 16) : 1, GS = (S >= 3) ? G : 16;  // lanes of a group, features of a lane group
+  constexpr int PHF = (S >= 3) ? (S - 1) : 1;
+  constexpr float kNorm = 1.0f / (float)(1 << S);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int nwaves = blockDim.x >> 6;
+  int64_t row = blockIdx.x;
+  if constexpr (MODE == CONVROT_PREP_FP6 || MODE == CONVROT_PREP_INT8_BLOCKED) {  // as prep_kernel
+    const int64_t run = ((int64_t)gridDim.x / (8 * 16)) * 16;
+    if (row < 8 * run) row = (row & 7) * run + (row >> 3);
+  }
+  const int chunks = K >> 4;
+  const __amdgpu_buffer_rsrc_t xrow = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const char*)x + row * (PRO == kProGelu ? pa.x_stride : (int64_t)K) * 2), (short)0,
+      (PRO == kProGelu ? K - pa.head_features : K) * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t hrow = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(PRO == kProGelu && pa.head_features ? (const char*)pa.head + row * pa.head_stride * 2
+                                                  : (const char*)x),
+      (short)0, PRO == kProGelu ? pa.head_features * 2 : 0, 0x00020000);
+  uint32_t* wave_lds = lds + wave * kPkRegion;
+  uint32_t* region = wave_lds + (lane / LG) * pk_off(G);
+  const int p = lane % LG;
+  const Matrices mat = matrices(lane);
+
+  uint32_t h[NI][8];
+  // ---- producer: x's 16 values of an iteration, past the row end zeros
+  float mean = 0.0f, rstd = 0.0f;
+  const int64_t vrow = PRE ? row / pa.rows_per_vector : 0;
+  auto load = [&](int it, uint32_t (&v)[8]) {
+    const int f0 = ((wave * NI + it) * 64 + lane) * 16;
+    if (PRO == kProGelu && f0 < pa.head_features) {  // head_features % 16 == 0: a chunk lies in one segment
+      pk_load16(hrow, (uint32_t)f0 * 2u, v);
+    } else {
+      pk_load16(xrow, (uint32_t)(f0 - (PRO == kProGelu ? pa.head_features : 0)) * 2u, v);
+    }
+  };
+  auto produce = [&](int it, uint32_t (&v)[8]) {
+    const int chunk = (wave * NI + it) * 64 + lane;
+    if constexpr (PRO == kProGelu) {
+      if (chunk * 16 >= pa.head_features) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          // the float32 result is rounded on its own, as the oracle does (no
+          // multiply-and-narrow folding into one v_fma_mix for f16)
+          float lo = gelu_tanh32(pk_lo<DT>(v[i])), hi = gelu_tanh32(pk_hi<DT>(v[i]));
+          asm volatile("" : "+v"(lo), "+v"(hi));
+          v[i] = pk_make<DT>(lo, hi);
+        }
+      }
+    } else if constexpr (PRE) {
+      if (chunk < chunks) {  // padding stays zero (whole groups lie past K)
+        const __amdgpu_buffer_rsrc_t shrow = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)((const char*)pa.shift + vrow * K * 2), (short)0, K * 2, 0x00020000);
+        const __amdgpu_buffer_rsrc_t scrow = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)((const char*)pa.scale + vrow * K * 2), (short)0, K * 2, 0x00020000);
+        uint32_t sh[8], sc[8];
+        pk_load16(shrow, (uint32_t)chunk * 32u, sh);
+        pk_load16(scrow, (uint32_t)chunk * 32u, sc);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          float plo = (pk_lo<DT>(v[i]) - mean) * rstd, phi = (pk_hi<DT>(v[i]) - mean) * rstd;
+          asm volatile("" : "+v"(plo), "+v"(phi));  // rounded before the dtype rounding, as in prep_kernel
+          const float lo = rnd<DT>(rnd<DT>(1.0f + pk_lo<DT>(sc[i])) * rnd<DT>(plo)) + pk_lo<DT>(sh[i]);
+          const float hi = rnd<DT>(rnd<DT>(1.0f + pk_hi<DT>(sc[i])) * rnd<DT>(phi)) + pk_hi<DT>(sh[i]);
+          v[i] = pk_make<DT>(lo, hi);
+        }
+      }
+    }
+  };
+
+  // every iteration's loads go out first: the wave's share of the row in flight at once
+#pragma unroll
+  for (int it = 0; it < NI; ++it) load(it, h[it]);
+  if constexpr (PRE) {
+    const int real_blocks = (chunks + 63) >> 6;
+#pragma unroll
+    for (int it = 0; it < NI; ++it) {
+      const int block = wave * NI + it;
+      __builtin_amdgcn_sched_barrier(0);
+      double b1 = 0.0, b2 = 0.0;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const double d = (double)(j & 1 ? pk_hi<DT>(h[it][j >> 1]) : pk_lo<DT>(h[it][j >> 1]));
+        b1 += d;
+        b2 = __builtin_fma(d, d, b2);  // the square is exact
+      }
+      b1 = wave_sum_f64(b1);
+      b2 = wave_sum_f64(b2);
+      if (lane == 0 && block < real_blocks) {
+        block_moments[block][0] = b1;
+        block_moments[block][1] = b2;
+      }
+    }
+    __syncthreads();
+    double s1 = 0.0, s2 = 0.0;
+    for (int b = 0; b < real_blocks; ++b) {
+      s1 += block_moments[b][0];
+      s2 += block_moments[b][1];
+    }
+    const double m64 = s1 / (double)K;
+    double var = s2 / (double)K - m64 * m64;
+    var = var > 0.0 ? var : 0.0;
+    mean = (float)m64;
+    rstd = (float)(1.0 / sqrt(var + (double)pa.eps));
+  }
+
+  uint32_t pmax = 0;
+#pragma unroll
+  for (int it = 0; it < NI; ++it) {
+    if constexpr (PRO != kProPlain) __builtin_amdgcn_sched_barrier(0);  // one iteration's operands in registers at a time
+    produce(it, h[it]);
+    pk_rotate16<DT, S>(mat, h[it], region, p);
+    if constexpr (DT == kF16 && MODE != CONVROT_PREP_ROTATE) {
+      const f16x2 norm = {(_Float16)kNorm, (_Float16)kNorm};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) h[it][i] = as_u32(as_f16(h[it][i]) * norm);
+    }
+    pmax = pk_absmax(pmax, h[it]);
+  }
+
+  // ---- row scale (core.py:154-156)
+  RowScale<DT> rs{};
+  constexpr uint32_t kInf = DT == kBF16 ? 0x7f80u : 0x7c00u;
+  const uint32_t top = __float_as_uint(wave_max_nonneg(__uint_as_float(max(pmax & 0xffffu, pmax >> 16))));
+  bool bad = top >= kInf;  // this wave holds an infinity or NaN (wave-uniform)
+  float amax = DT == kBF16 ? bf16_lo(top) : (float)as_f16(top).x;
+  if (bad) {  // once more by the float32 butterfly, as prep_kernel does (absmax3 passes over NaN)
+    float exact = 0.0f;
+#pragma unroll 1
+    for (int it = 0; it < NI; ++it) {
+      uint32_t w[8];
+      load(it, w);
+      produce(it, w);
+      pk_rotate16<DT, S, true>(mat, w, region, p);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if constexpr (DT == kF16 && MODE != CONVROT_PREP_ROTATE)
+          w[i] = pk_make<DT>(pk_lo<DT>(w[i]) * kNorm, pk_hi<DT>(w[i]) * kNorm);
+        exact = absmax3(exact, pk_lo<DT>(w[i]), pk_hi<DT>(w[i]));
+      }
+#pragma unroll
+      for (int k = 0; k < NI; ++k)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) h[k][i] = k == it ? w[i] : h[k][i];
+    }
+    amax = wave_max_nonneg(exact);
+  }
+  if constexpr (MODE != CONVROT_PREP_ROTATE) {
+    if (nwaves > 1) {
+      if (lane == 0) wave_max[wave] = amax;
+      __syncthreads();
+      amax = wave_max[0];
+      for (int w = 1; w < nwaves; ++w) amax = fmaxf(amax, wave_max[w]);
+    }
+    rs = row_scale<DT>(amax, kNorm);
+    if (wave == 0 && lane == 0) scales[row] = rs.scale;
+    bad |= !(rs.scale < __builtin_inff());
+  }
+  const float finv = DT == kF16 && rs.scale > 0.0f ? 1.0f / rs.scale : 0.0f;
+
+  // ---- quantize + store, phase-final layout
+#pragma unroll
+  for (int it = 0; it < NI; ++it) {
+    const int block = wave * NI + it;
+    const int chunk = block * 64 + lane;
+    if (chunk >= chunks) continue;
+    const uint32_t (&v)[8] = h[it];
+    float ratio[16];  // unrounded where they are packed next (FP6)
+    if constexpr (MODE != CONVROT_PREP_ROTATE) {
+      if (DT == kF16 && bad) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          ratio[2 * i] = code_ratio<DT>(pk_lo<DT>(v[i]), rs), ratio[2 * i + 1] = code_ratio<DT>(pk_hi<DT>(v[i]), rs);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float r = i & 1 ? pk_hi<DT>(v[i >> 1]) : pk_lo<DT>(v[i >> 1]);
+          ratio[i] = DT == kBF16 ? r * rs.inv : f16_quotient(r, rs.scale, finv);
+          if constexpr (MODE != CONVROT_PREP_FP6) ratio[i] = rnd<DT>(ratio[i]);
+        }
+      }
+    }
+    const int64_t mblocks = ((int64_t)gridDim.x + 15) >> 4;
+    if constexpr (MODE == CONVROT_PREP_FP6) {
+      // 16 consecutive features (a group's half stream, 12 bytes) are 4 runs
+      // of 4: the lane's own 4 runs for groups up to 16, else run r of the 4
+      // lanes of a quad (lane k holding features 4k .. 4k+3 of it), which
+      // lane r of the quad gathers through the wave's LDS region.
+      uint32_t d0, d1, d2;
+      const int qb = lane & ~3, k = lane & 3;
+      uint32_t* xr = wave_lds;
+      uint32_t hp[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        hp[i] = pk_make<DT>(ratio[2 * i], ratio[2 * i + 1]);
+        if constexpr (DT == kBF16) hp[i] = zero_code_sign_fix(hp[i]);
+        else hp[i] = bad ? hp[i] : f16_clamp_sign_fix(hp[i]);
+      }
+      if constexpr (S >= 3) {
+        wave_lds_fence();
+#pragma unroll
+        for (int run = 0; run < 4; ++run)
+          *(uint2*)(xr + (qb + run) * 8 + 2 * k) = make_uint2(hp[2 * run], hp[2 * run + 1]);
+        wave_lds_fence();
+        const uint4 g0 = *(const uint4*)(xr + (qb + k) * 8), g1 = *(const uint4*)(xr + (qb + k) * 8 + 4);
+        hp[0] = g0.x, hp[1] = g0.y, hp[2] = g0.z, hp[3] = g0.w;
+        hp[4] = g1.x, hp[5] = g1.y, hp[6] = g1.z, hp[7] = g1.w;
+      }
+      if (DT == kF16 && bad) {  // NaN ratios: the codes of prep_kernel's float16
+        uint32_t pc[4];
+#pragma unroll
+        for (int run = 0; run < 4; ++run) {
+          float r[4];
+          r[0] = pk_lo<DT>(hp[2 * run]), r[1] = pk_hi<DT>(hp[2 * run]);
+          r[2] = pk_lo<DT>(hp[2 * run + 1]), r[3] = pk_hi<DT>(hp[2 * run + 1]);
+          pc[run] = fp6_piece(code_bits(fabsf(r[0])), code_bits(fabsf(r[1])), code_bits(fabsf(r[2])),
+                              code_bits(fabsf(r[3])), r[0], r[1], r[2], r[3]);
+        }
+        d0 = pc[0] | (pc[1] << 24);
+        d1 = (pc[1] >> 8) | (pc[2] << 16);
+        d2 = (pc[2] >> 16) | (pc[3] << 8);
+      } else {
+        pk_fp6_fields16<DT>(hp, d0, d1, d2);
+      }
+      int fh;  // first feature (in the row) of the half this lane writes
+      if constexpr (S >= 3) fh = block * 1024 + (lane / LG) * GS + run_index<S, PHF>(p & ~3, k);
+      else fh = block * 1024 + lane * 16;
+      uint8_t* blk = (uint8_t*)out + ((int64_t)(fh >> 7) * mblocks + (row >> 4)) * 1536;
+      const int L = ((fh >> 5) & 3) * 16 + (int)(row & 15);
+      // The two halves of a 32-feature group share slot L: 12 bytes of the
+      // first, then the second's first dword (its other 8 bytes go to the
+      // block's tail).  They sit in lanes kPair apart (bit 4 of fh is lane bit
+      // 2 for groups of 256 and 1024, lane bit 0 otherwise), so the first lane
+      // writes the whole 16-byte slot: two stores a pair instead of three.
+      // Both lanes of a pair are past the row end or neither (K % 128 == 0).
+      constexpr int kPair = (S == 4 || S == 5) ? 4 : 1;
+      const uint32_t d0_second = (uint32_t)__shfl_down((int)d0, kPair);
+      if ((fh & 16) == 0) {
+        *(uint4*)(blk + 16 * L) = make_uint4(d0, d1, d2, d0_second);
+      } else {
+        *(uint2*)(blk + 1024 + 8 * L) = make_uint2(d1, d2);
+      }
+    } else {
+#pragma unroll
+      for (int run = 0; run < 4; ++run) {
+        const int fr = block * 1024 + (lane / LG) * GS + run_index<(S >= 3 ? S : 3), PHF>(p, run);
+        const int64_t f = row * K + fr;
+        if constexpr (MODE == CONVROT_PREP_ROTATE) {
+          // core.py:94 -- y / sqrt(G), rounded to the dtype
+          const f16x2 norm = {(_Float16)kNorm, (_Float16)kNorm};
+          *(uint2*)((uint16_t*)out + f) =
+              make_uint2(as_u32(as_f16(v[2 * run]) * norm), as_u32(as_f16(v[2 * run + 1]) * norm));
+        } else {
+          const uint32_t q0 = code_bits(ratio[4 * run]), q1 = code_bits(ratio[4 * run + 1]),
+                         q2 = code_bits(ratio[4 * run + 2]), q3 = code_bits(ratio[4 * run + 3]);
+          if constexpr (MODE == CONVROT_PREP_INT8_BLOCKED) {
+            uint8_t* blk = (uint8_t*)out + ((int64_t)(fr >> 7) * mblocks + (row >> 4)) * 2048;
+            *(uint32_t*)(blk + (fr & 16) * 64 + (((fr >> 5) & 3) * 16 + (int)(row & 15)) * 16 + (fr & 15)) =
+                gather_bytes(q0, q1, q2, q3);
+          } else if constexpr (MODE == CONVROT_PREP_INT8) {
+            ((uint32_t*)out)[f >> 2] = gather_bytes(q0, q1, q2, q3);
+          } else {
+            ((uint16_t*)out)[f >> 2] = (uint16_t)gather_nibbles(q0, q1, q2, q3);
+          }
+        }
+      }
+    }
+  }
+}
+
+// Whether prep16_kernel prepares these rows.
+constexpr bool prep_packed(int dtype, int log4g, int mode) {
+  return log4g >= 1 && (dtype == kF16 || (dtype == kBF16 && mode != CONVROT_PREP_ROTATE));
+}
+
 // The producer of a launch and its arguments.
 struct Modulation {
   int producer;  // kProPlain, kProModulate or kProGelu
@@ -439,16 +980,29 @@ struct Modulation {
 template <int DT, int S, int NI, int MODE>
 hipError_t launch_prep_t(const void* x, void* out, float* scales, int64_t rows, int K, int waves,
                          const Modulation& mod, hipStream_t stream) {
-  const size_t lds_bytes = (S >= 3) ? (size_t)waves * kRegionFloats * sizeof(float) : 0;
-  if (mod.producer == kProModulate)
-    hipLaunchKernelGGL((prep_kernel<DT, S, NI, MODE, kProModulate>), dim3((unsigned)rows), dim3(64 * waves),
-                       lds_bytes, stream, x, out, scales, K, mod.args);
-  else if (mod.producer == kProGelu)
-    hipLaunchKernelGGL((prep_kernel<DT, S, NI, MODE, kProGelu>), dim3((unsigned)rows), dim3(64 * waves),
-                       lds_bytes, stream, x, out, scales, K, mod.args);
-  else
-    hipLaunchKernelGGL((prep_kernel<DT, S, NI, MODE, kProPlain>), dim3((unsigned)rows), dim3(64 * waves),
-                       lds_bytes, stream, x, out, scales, K, mod.args);
+  constexpr bool kPacked = prep_packed(DT, S, MODE);
+  const auto launch = [&](void (*kernel)(const void*, void*, float*, int, ProducerArgs), int region) {
+    const size_t lds_bytes = S >= 3 ? (size_t)waves * (size_t)region * 4 : 0;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(64 * waves), lds_bytes, stream, x, out, scales, K, mod.args);
+  };
+  if constexpr (kPacked) {
+    // bf16 rows of four blocks a wave behind the modulated producer spill on the packed kernel (8800 x 16384:
+    // 193 us against 174 on the other)
+    if (mod.producer == kProModulate) {
+      if constexpr (DT == kBF16 && NI == 4) launch(prep_kernel<DT, S, NI, MODE, kProModulate>, kRegionFloats);
+      else launch(prep16_kernel<DT, S, NI, MODE, kProModulate>, kPkRegion);
+    } else if (mod.producer == kProGelu) {
+      launch(prep16_kernel<DT, S, NI, MODE, kProGelu>, kPkRegion);
+    } else {
+      launch(prep16_kernel<DT, S, NI, MODE, kProPlain>, kPkRegion);
+    }
+  } else if constexpr (S == 0) {  // no rotation: the plain producer only
+    launch(prep_kernel<DT, S, NI, MODE, kProPlain>, kRegionFloats);
+  } else {
+    if (mod.producer == kProModulate) launch(prep_kernel<DT, S, NI, MODE, kProModulate>, kRegionFloats);
+    else if (mod.producer == kProGelu) launch(prep_kernel<DT, S, NI, MODE, kProGelu>, kRegionFloats);
+    else launch(prep_kernel<DT, S, NI, MODE, kProPlain>, kRegionFloats);
+  }
   return hipGetLastError();
 }
 
@@ -496,8 +1050,11 @@ hipError_t launch_prep_s(int s, int ni, int mode, const void* x, void* out, floa
 // Pick (iterations per wave, waves per row) so that 1024*NI*W covers K with
 // the fewest idle 1024-feature blocks; NI in {3, 4, 1}, W <= 16.  Few rows
 // (M <= 2048) take one iteration per wave and more waves per row instead, so
-// that enough waves are in flight to cover the load latency.
-bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out) {
+// that enough waves are in flight to cover the load latency; the packed kernel
+// only up to 12288 blocks in all (1536 x 15360, one iteration -> four: 21.4 ->
+// 18.7 us, modulated 39.1 -> 34.2; the other kernel and the GELU producer gain
+// nothing there: `packed` is false for them).
+bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out, bool packed) {
   const int64_t blocks = (K + 1023) / 1024;
   {  // tuning override: force the iterations per wave
     const int ni = tuning(kTunePrepNi);
@@ -510,7 +1067,7 @@ bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out) {
       }
     }
   }
-  if (rows <= 2048 && blocks <= kMaxWaves) {
+  if (rows <= 2048 && blocks <= kMaxWaves && !(packed && rows * blocks > 12288)) {
     *ni_out = 1;
     *waves_out = (int)blocks;
     return true;
@@ -551,7 +1108,7 @@ namespace {
 hipError_t launch_prep_any(const void* x, int dtype, int64_t rows, int64_t K, int log4g, int mode, void* out,
                            float* scales, const Modulation& mod, hipStream_t stream) {
   int ni = 0, waves = 0;
-  if (!prep_plan(rows, K, &ni, &waves)) return hipErrorInvalidValue;
+  if (!prep_plan(rows, K, &ni, &waves, prep_packed(dtype, log4g, mode) && mod.producer != kProGelu)) return hipErrorInvalidValue;
   if (rows == 0) return hipSuccess;
   switch (dtype) {
     case kF32: return launch_prep_s<kF32>(log4g, ni, mode, x, out, scales, rows, (int)K, waves, mod, stream);

@@ -1,0 +1,112 @@
+"""GPU parity: the preparation of 16-bit activations on packed registers, where it can go wrong."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from _util import from_dev, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(orc, dev, x16, dtype, G):
+    """Codes and scales of the int8, packed, blocked and FP6 outputs against the oracle's."""
+    from convrot_mlx_amd import _native as nat
+    from convrot_mlx_amd import core
+
+    M, K = x16.shape
+    codes, scales = orc.prepare_codes(x16, dtype, G)
+    x = to_dev(x16, dtype, dev)
+    got, s = core._prepare(x, G, nat.PREP_INT8)
+    assert np.array_equal(from_dev(got), codes) and np.array_equal(from_dev(s), scales)
+    got, s = core._prepare(x, G, nat.PREP_PACKED)
+    assert np.array_equal(from_dev(got), orc.pack_signed_int4(codes)) and np.array_equal(from_dev(s), scales)
+    if K % 128 == 0:
+        got, s = core._prepare(x, G, nat.PREP_FP6)
+        assert np.array_equal(orc.fp6_to_codes(from_dev(got), M, K), codes) and np.array_equal(from_dev(s), scales)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("G", [4, 16, 64, 256, 1024])
+@pytest.mark.parametrize("ni", [1, 3, 4])
+def test_magnitudes(orc, dev, tuning, dtype, G, ni):
+    """Every group size and iteration count on rows of every magnitude: the format's smallest denormals,
+    values 2^20 apart in one group (sums that round), the largest that stay finite, zeros of both signs."""
+    tuning.set("prep_ni", ni)
+    rng = np.random.default_rng(G + ni)
+    K = 5120
+    top = 2.0 ** (90 if dtype == "bfloat16" else 4)
+    rows = [rng.normal(size=K) * s for s in (1.0, top, 2.0 ** -24, 2.0 ** -20, 2.0 ** -14)]
+    rows.append(rng.normal(size=K) * 2.0 ** rng.integers(-20, 3, size=K))
+    rows.append(np.where(rng.random(K) < 0.5, -0.0, 0.0))
+    rows.append(rng.integers(-3, 4, size=K) * 2.0 ** -24)
+    if dtype == "bfloat16":
+        rows += [rng.normal(size=K) * 2.0 ** -130, rng.integers(-2, 3, size=K) * 2.0 ** -133]
+    with np.errstate(over="ignore"):
+        x16 = orc.from_f32(np.array(rows, dtype=np.float32), dtype)
+    _check(orc, dev, x16, dtype, G)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("mode", ["int8", "fp6", "blocked", "packed"])
+def test_nonfinite_rows(dev, dtype, mode):
+    """Infinities, NaN and sums that overflow: the bits of the float32 kernel's arithmetic (a float16 or
+    bfloat16 row prepared without rotation after an eager rotation in the dtype), rows beside them untouched."""
+    from convrot_mlx_amd import _native as nat
+    from convrot_mlx_amd import core
+
+    kind = {"int8": nat.PREP_INT8, "fp6": nat.PREP_FP6, "blocked": nat.PREP_INT8_BLOCKED, "packed": nat.PREP_PACKED}[mode]
+    dt = {"bfloat16": torch.bfloat16, "float16": torch.float16}[dtype]
+    M, K, G = 6, 4096, 256
+    x = torch.randn(M, K, device=dev)
+    big = 3e38 if dtype == "bfloat16" else 6e4
+    x[1, 70], x[2, 3000], x[2, 3001], x[3, :] = float("inf"), float("-inf"), float("inf"), big
+    x[4, 5], x[4, 2000] = float("nan"), 9.0
+    x = x.to(dt)
+    got, scales = core._prepare(x, G, kind)
+
+    def rotate(v):  # the eager butterfly, every sum rounded to the dtype
+        stride = 1
+        while stride < G:
+            a, b, c, d = v.reshape(M, K // (4 * stride), 4, stride).unbind(2)
+            v = torch.stack([a + b + c - d, a + b - c + d, a - b + c + d, -a + b + c + d], 2).reshape(M, K)
+            stride *= 4
+        return (v.float() / 16).to(dt)
+
+    want, want_scales = core._prepare(rotate(x), 1, kind | nat.PREP_NO_ROTATE)
+    assert torch.equal(scales.nan_to_num(1.5), want_scales.nan_to_num(1.5))
+    if mode == "fp6":  # [kb, 1, 16 bytes of a (q, row) slot]; a NaN's field has the NaN's sign, which torch's may not
+        rows = lambda t: t[:, 0, :1024].reshape(K // 128, 4, 16, 16)[:, :, :M]  # noqa: E731
+        nan = torch.isnan(rotate(x).float() / scales[:, None])
+        clean = ~nan.reshape(M, K // 128, 4, 32).any(-1).permute(1, 2, 0)
+        assert torch.equal(rows(got)[clean], rows(want)[clean])
+    elif mode == "blocked":
+        rows = lambda t: t.reshape(K // 128, 2, 4, 16, 16)[:, :, :, :M]  # noqa: E731
+        assert torch.equal(rows(got), rows(want))
+    else:
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_gelu_every_value(orc, dev, dtype):
+    """Every 16-bit input with finite sums through the GELU producer: the oracle's codes (the reciprocal and the
+    exponent arithmetic at every significand and range), and a head in front."""
+    from convrot_mlx_amd import _native as nat
+    from convrot_mlx_amd import core
+
+    bits = np.arange(65536, dtype=np.uint16)
+    # below an eighth of the largest value, so that the sums of a group stay finite
+    bits = bits[np.abs(orc.to_f32(bits, dtype)) < (2.0 ** 124 if dtype == "bfloat16" else 2.0 ** 12)]
+    order = np.argsort(np.abs(orc.to_f32(bits, dtype)), kind="stable")  # rows of like magnitudes: codes of all of them
+    bits = bits[order][: bits.size // 256 * 256].reshape(-1, 256)
+    head = np.ascontiguousarray(bits[:, :64])
+    x16 = orc.gelu_producer_rows(None, bits, dtype)
+    codes, scales = orc.prepare_codes(x16, dtype, 4)
+    got, s = core._prepare_gelu(to_dev(bits, dtype, dev), None, 4, nat.PREP_INT8)
+    assert np.array_equal(from_dev(got), codes) and np.array_equal(from_dev(s), scales)
+    x16 = orc.gelu_producer_rows(head, bits, dtype)
+    codes, scales = orc.prepare_codes(x16, dtype, 64)
+    got, s = core._prepare_gelu(to_dev(bits, dtype, dev), to_dev(head, dtype, dev), 64, nat.PREP_PACKED)
+    assert np.array_equal(from_dev(got), orc.pack_signed_int4(codes)) and np.array_equal(from_dev(s), scales)
