@@ -145,7 +145,8 @@ def set_tuning(name: str, value: str | None) -> None:
     gemm_sk_min, gemm_no_dma, gemm_smallm_max, w4a4_smallm_cfg (A/B/C/F), w4a16_cfg
     (A/B/C/D/E/F, S: split K, T), w4a16_tile ("BMxBN"), prep_ni (1/3/4), sk_spin_limit, gemm_persist (0: never;
     G: always, on G workgroups), gemm_mfma32 (0/1), fp6_tile ("BMxBN": 256x256, 256x224, 128x256, 128x192, 128x128),
-    linear_rows_cfg (1/2/3/5/16), w4a4_midm_cfg (10 * row tiles + weight tiles)."""
+    linear_rows_cfg (1/2/3/5/16), w4a4_midm_cfg (10 * row tiles + weight tiles),
+    fp6_split (1/2/4: parts of each 256x256 FP6 tile past the whole rounds)."""
     check(load().convrot_set_tuning(name.encode(), None if value is None else str(value).encode()))
 
 

@@ -98,7 +98,7 @@ int convrot_set_tuning(const char* name, const char* value) {
                 {"prep_ni", kTunePrepNi},             {"sk_spin_limit", kTuneSkSpinLimit},
                 {"gemm_persist", kTuneGemmPersist},   {"gemm_mfma32", kTuneGemmMfma32},
                 {"fp6_tile", kTuneFp6Tile},           {"linear_rows_cfg", kTuneRowsCfg},
-                {"w4a4_midm_cfg", kTuneMidmCfg}};
+                {"w4a4_midm_cfg", kTuneMidmCfg},      {"fp6_split", kTuneFp6Split}};
   int key = -1;
   for (const auto& n : kNames)
     if (strcmp(n.name, name) == 0) key = n.key;
@@ -135,6 +135,10 @@ int convrot_set_tuning(const char* name, const char* value) {
       case kTuneRowsCfg:
         v = atoi(value);
         good = v == 1 || v == 2 || v == 3 || v == 5 || v == 16;
+        break;
+      case kTuneFp6Split:
+        v = atoi(value);
+        good = v == 1 || v == 2 || v == 4;
         break;
       case kTuneMidmCfg:
         v = atoi(value);

@@ -30,6 +30,7 @@ enum TuneKey : int {
   kTuneFp6Tile,          // FP6 W4A4 tile: bm | bn << 10
   kTuneRowsCfg,          // few-row linear: weight tiles a workgroup (1, 2, 3, 5), or 16: one tile on 16 waves
   kTuneMidmCfg,          // W4A4 kernel of blocked codes: 10 * row tiles + weight tiles of a workgroup
+  kTuneFp6Split,         // FP6 256x256 tiles past the whole rounds: as 1, 2 or 4 workgroups
   kTuneCount
 };
 int tuning(TuneKey key);

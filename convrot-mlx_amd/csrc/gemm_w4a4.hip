@@ -1764,24 +1764,16 @@ struct Fp6Engine {
   }
 };
 
-// The FP6 GEMM, one BM x BN tile per workgroup of 2 WN waves, with the
+// One BM x BN output tile at (m0, n0) by a workgroup of 2 WN waves, with the
 // epilogue of every W4A4 kernel (16-bit or float32 outputs, optional gated
-// residual).  Two waves a SIMD for the 128 x 128 tile (two workgroups a CU)
-// and the 8-wave tiles.
-template <int BM, int BN, int ODT, bool CW, int WN>
-__global__ __launch_bounds__(WN * 128) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2 : 1, BM * BN <= 128 * 128 || WN == 4 ? 2 : 1))) void w4a4_gemm_fp6_kernel(
-    const uint8_t* __restrict__ act, const float* __restrict__ xscales, const uint8_t* __restrict__ wq,
-    const float* __restrict__ wscales, const float* __restrict__ bias, void* __restrict__ out, int M, int N,
-    int K, int nblocks, int tiles_m, int tiles_n, GatedResidual gr) {
-  using E = Fp6Engine<BM, BN, CW, WN>;
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[E::SMEM_BYTES];
+// residual).
+template <class E, int ODT>
+__device__ __forceinline__ void fp6_tile_at(uint8_t* smem, const uint8_t* __restrict__ act,
+                                            const float* __restrict__ xscales, const uint8_t* __restrict__ wq,
+                                            const float* __restrict__ wscales, const float* __restrict__ bias,
+                                            void* __restrict__ out, int M, int N, int K, int nblocks, int m0, int n0,
+                                            const GatedResidual& gr) {
   E e(smem);
-  const int tiles = tiles_m * tiles_n;
-  int logical = blockIdx.x;
-  const int per_xcd = tiles / kXcds;
-  if (logical < per_xcd * kXcds) logical = (logical % kXcds) * per_xcd + logical / kXcds;
-  int m0, n0;
-  tile_origin(logical, tiles_m, tiles_n, BM, BN, m0, n0);
   const int kblocks = K / 128;
   e.set_tile(act, wq, M, K, nblocks, m0, n0);
   e.issue_epi(xscales, wscales, bias, M, N, m0, n0);
@@ -1797,6 +1789,54 @@ __global__ __launch_bounds__(WN * 128) __attribute__((amdgpu_waves_per_eu(WN == 
                                        n0 + e.wn * E::TN, M, N, (const float*)(smem + E::EPI_OFF),
                                        (const float*)(smem + E::WS_OFF), (const float*)(smem + E::BIAS_OFF), out, gr,
                                        m0, n0);
+}
+
+// The FP6 GEMM, one BM x BN tile per workgroup of 2 WN waves.  Two waves a SIMD
+// for the 128 x 128 tile (two workgroups a CU) and the 8-wave tiles.
+template <int BM, int BN, int ODT, bool CW, int WN>
+__global__ __launch_bounds__(WN * 128) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2 : 1, BM * BN <= 128 * 128 || WN == 4 ? 2 : 1))) void w4a4_gemm_fp6_kernel(
+    const uint8_t* __restrict__ act, const float* __restrict__ xscales, const uint8_t* __restrict__ wq,
+    const float* __restrict__ wscales, const float* __restrict__ bias, void* __restrict__ out, int M, int N,
+    int K, int nblocks, int tiles_m, int tiles_n, GatedResidual gr) {
+  using E = Fp6Engine<BM, BN, CW, WN>;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[E::SMEM_BYTES];
+  const int tiles = tiles_m * tiles_n;
+  int logical = blockIdx.x;
+  const int per_xcd = tiles / kXcds;
+  if (logical < per_xcd * kXcds) logical = (logical % kXcds) * per_xcd + logical / kXcds;
+  int m0, n0;
+  tile_origin(logical, tiles_m, tiles_n, BM, BN, m0, n0);
+  fp6_tile_at<E, ODT>(smem, act, xscales, wq, wscales, bias, out, M, N, K, nblocks, m0, n0, gr);
+}
+
+// 256 x 256 tiles whose last round is a part of one: the first `whole` tiles
+// (whole rounds) run as they are, each of the others as SUB workgroups, 128 x 256
+// (SUB 2) or 128 x 128 (SUB 4), that fill the CUs the last round would leave
+// idle.  The parts come last in the grid, so that they are dispatched last; a
+// part outside the output ends at once.  The plan's rule is beside fp6_tile.
+template <int ODT, int SUB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void w4a4_gemm_fp6_mixed_kernel(
+    const uint8_t* __restrict__ act, const float* __restrict__ xscales, const uint8_t* __restrict__ wq,
+    const float* __restrict__ wscales, const float* __restrict__ bias, void* __restrict__ out, int M, int N,
+    int K, int nblocks, int tiles_m, int tiles_n, int whole, GatedResidual gr) {
+  using E = Fp6Engine<256, 256, true, 4>;
+  using P = Fp6Engine<128, SUB == 2 ? 256 : 128, true, 4>;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[E::SMEM_BYTES > P::SMEM_BYTES ? E::SMEM_BYTES : P::SMEM_BYTES];
+  int b = blockIdx.x;
+  int m0, n0;
+  if (b < whole) {  // a multiple of the XCDs
+    tile_origin((b % kXcds) * (whole / kXcds) + b / kXcds, tiles_m, tiles_n, 256, 256, m0, n0);
+    fp6_tile_at<E, ODT>(smem, act, xscales, wq, wscales, bias, out, M, N, K, nblocks, m0, n0, gr);
+    return;
+  }
+  b -= whole;
+  const int parts = (tiles_m * tiles_n - whole) * SUB, per_xcd = parts / kXcds;
+  if (b < per_xcd * kXcds) b = (b % kXcds) * per_xcd + b / kXcds;
+  tile_origin(whole + b / SUB, tiles_m, tiles_n, 256, 256, m0, n0);
+  m0 += 128 * (b & 1);
+  if constexpr (SUB == 4) n0 += 128 * ((b >> 1) & 1);
+  if (m0 >= M || n0 >= N) return;  // the whole workgroup
+  fp6_tile_at<P, ODT>(smem, act, xscales, wq, wscales, bias, out, M, N, K, nblocks, m0, n0, gr);
 }
 
 // ---- stream-K
@@ -2542,11 +2582,26 @@ namespace {
 struct Fp6Tile {
   int bm, bn;
   double rel;
+  int sub = 1;  // parts of each tile past the whole rounds (256 x 256, compact weights)
 };
 constexpr Fp6Tile kFp6Tiles[5] = {{256, 256, 0.86}, {256, 224, 0.9}, {128, 256, 0.58}, {128, 128, 0.43}, {128, 192, 0.54}};
+// Where the 256 x 256 tiles leave a part of a round over, every whole round runs
+// as it is and each leftover tile as 2 or 4 workgroups of 8 waves, on the
+// compact weights: the last round then takes a part's time (kFp6Parts) instead of
+// a tile's, as long as the parts fit one round: up to 64 leftover tiles go in
+// four, up to 128 in two.  The linear with its preparation, as tiles | in two | in
+// four (us, medians of 5 x 30 calls in turn):
+//   8800 x 16384 -> 4096, 48 over two rounds:   394.8 | 370.6 | 367.1
+//   4608 x 3072 -> 3840, 14 over one:            52.2 |  53.3 |  48.7
+//   6144 x 2048 -> 6144, 64 over two:            70.1 |  65.7 |  63.6
+//   2304 x 12288 -> 9216, 68 over one:          172.3 | 149.6 | 171.7
+//   4608 x 3072 -> 12288, 96 over three:        114.6 | 109.3 | 115.1
+//   8192 x 3072 -> 3072, 128 over one:           68.0 |  63.2 |  69.2
+//   3072 x 3072 -> 9216, 176 over one:           60.2 |  70.0 |  71.7 (left as tiles)
+constexpr double kFp6Parts[2] = {0.58, 0.43};
 
-Fp6Tile fp6_tile(int64_t M, int64_t N) {
-  const int forced = tuning(kTuneFp6Tile);
+Fp6Tile fp6_tile(int64_t M, int64_t N, bool compact) {
+  const int forced = tuning(kTuneFp6Tile), split = tuning(kTuneFp6Split);
   if (forced >= 0)
     for (const Fp6Tile& t : kFp6Tiles)
       if ((forced & 1023) == t.bm && (forced >> 10) == t.bn) return t;
@@ -2562,12 +2617,34 @@ Fp6Tile fp6_tile(int64_t M, int64_t N) {
     // rounds of two a CU on: 1536 x 3072 -> 12288, 1152 tiles, 40.8 us
     // against 44.5 on 128 x 192); fewer tiles keep the rounded model.
     if (t.bm == 128 && t.bn == 128 && tiles >= 4 * cus) cost = (double)tiles / (double)cus * 0.33;
+    int sub = 1;
+    if (compact && t.bm == 256 && t.bn == 256 && tiles > cus && cus % kXcds == 0) {
+      const int64_t rest = tiles % cus;
+      for (int i = 0; i < 2; ++i) {
+        const int s = 2 << i;
+        const double mixed = (double)(tiles / cus) * t.rel + kFp6Parts[i];
+        if (split >= 0 ? split == s && rest > 0 : rest > 0 && rest * s <= cus && mixed < cost) cost = mixed, sub = s;
+      }
+    }
+    if (split > 1 && sub == split) cost = 0.0;  // forced
     if (best_cost < 0 || cost < best_cost - 1e-9) {
       best = t;
+      best.sub = sub;
       best_cost = cost;
     }
   }
   return best;
+}
+
+template <int ODT, int SUB>
+hipError_t launch_fp6_mixed(const uint8_t* act6, const float* xscales, const uint8_t* w6, const float* wscales,
+                            const float* bias, int64_t M, int64_t N, int64_t K, void* out, const GatedResidual& gr,
+                            hipStream_t stream) {
+  const int tm = (int)((M + 255) / 256), tn = (int)((N + 255) / 256), cus = device_cus();
+  const int whole = tm * tn / cus * cus, parts = (tm * tn - whole) * SUB;
+  hipLaunchKernelGGL((w4a4_gemm_fp6_mixed_kernel<ODT, SUB>), dim3((unsigned)(whole + parts)), dim3(512), 0, stream, act6,
+                     xscales, w6, wscales, bias, out, (int)M, (int)N, (int)K, (int)((N + 15) / 16), tm, tn, whole, gr);
+  return hipGetLastError();
 }
 
 template <int BM, int BN, int ODT, bool CW>
@@ -2587,7 +2664,11 @@ template <int ODT, bool CW>
 hipError_t launch_fp6_t(const uint8_t* act6, const float* xscales, const uint8_t* w6, const float* wscales,
                         const float* bias, int64_t M, int64_t N, int64_t K, void* out, const GatedResidual& gr,
                         hipStream_t stream) {
-  const Fp6Tile t = fp6_tile(M, N);
+  const Fp6Tile t = fp6_tile(M, N, CW);
+  if constexpr (CW) {
+    if (t.sub == 2) return launch_fp6_mixed<ODT, 2>(act6, xscales, w6, wscales, bias, M, N, K, out, gr, stream);
+    if (t.sub == 4) return launch_fp6_mixed<ODT, 4>(act6, xscales, w6, wscales, bias, M, N, K, out, gr, stream);
+  }
   if (t.bm == 256 && t.bn == 224)
     return launch_fp6_tile<256, 224, ODT, CW>(act6, xscales, w6, wscales, bias, M, N, K, out, gr, stream);
   if (t.bm == 128 && t.bn == 128)
@@ -2619,7 +2700,7 @@ bool fp6_tile_known(int bm, int bn) {
 }
 
 void fp6_plan_tile(int64_t M, int64_t N, int* bm, int* bn) {
-  const Fp6Tile t = fp6_tile(M, N);
+  const Fp6Tile t = fp6_tile(M, N, true);
   *bm = t.bm;
   *bn = t.bn;
 }
