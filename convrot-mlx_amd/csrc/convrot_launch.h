@@ -42,7 +42,8 @@ bool w4a4_tile_known(int bm, int bn, int wm, int wn, int stages);
 bool fp6_tile_known(int bm, int bn);
 bool w4a16_tile_known(int bm, int bn);
 
-// The FP6 W4A4 tile the plan (and the fp6_tile override) picks for M x N.
+// The FP6 W4A4 tile the plan (and the fp6_tile override) picks for M x N on operand
+// blocks; compact weights may split the last round of a 256 x 256 grid instead.
 void fp6_plan_tile(int64_t M, int64_t N, int* bm, int* bn);
 
 bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out, bool packed);

@@ -2700,7 +2700,7 @@ bool fp6_tile_known(int bm, int bn) {
 }
 
 void fp6_plan_tile(int64_t M, int64_t N, int* bm, int* bn) {
-  const Fp6Tile t = fp6_tile(M, N, true);
+  const Fp6Tile t = fp6_tile(M, N, false);
   *bm = t.bm;
   *bn = t.bn;
 }
