@@ -185,8 +185,8 @@ struct MidmSplit {
 constexpr MidmSplit kMidmSplits[] = {{2, 1, 3, 0.3}, {2, 2, 2, 0.3}, {2, 3, 1, 1.2}, {2, 4, 1, 1.2}, {3, 1, 2, 0.3},
                                      {3, 2, 1, 1.2}, {3, 3, 1, 1.2}, {4, 3, 1, 1.2}, {5, 2, 1, 1.2}};
 
-double midm_cost(const MidmSplit& s, int64_t M, int64_t N, int64_t K) {
-  const int64_t cus = device_cus(), kblocks = (K + 127) / 128;
+double midm_cost(const MidmSplit& s, int64_t M, int64_t N, int64_t K, int64_t cus) {
+  const int64_t kblocks = (K + 127) / 128;
   const int64_t wgs = ((M + 15) / 16 + s.fm - 1) / s.fm * (((N + 15) / 16 + s.nb - 1) / s.nb);
   const int64_t full = wgs / (cus * s.per_cu), rest = wgs - full * cus * s.per_cu;
   const double shared = 1.0 + 0.7 * (s.per_cu - 1);
@@ -195,10 +195,13 @@ double midm_cost(const MidmSplit& s, int64_t M, int64_t N, int64_t K) {
   return ((double)full * shared + last) * (s.fixed + (double)((kblocks + kWaves - 1) / kWaves) * block);
 }
 
-const MidmSplit& midm_best(int64_t M, int64_t N, int64_t K) {
+// The best split and its cost.  `cus` comes from one device query: this runs on
+// every call of a layer.
+const MidmSplit& midm_best(int64_t M, int64_t N, int64_t K, int64_t cus, double* cost) {
   const MidmSplit* best = &kMidmSplits[0];
+  *cost = midm_cost(*best, M, N, K, cus);
   for (const MidmSplit& s : kMidmSplits)
-    if (midm_cost(s, M, N, K) < midm_cost(*best, M, N, K)) best = &s;
+    if (const double c = midm_cost(s, M, N, K, cus); c < *cost) best = &s, *cost = c;
   return *best;
 }
 
@@ -224,9 +227,12 @@ bool midm_preferred(int64_t M, int64_t N, int64_t K) {
     if (tuning(k) >= 0) return false;  // a kernel of row-major codes is asked for
   if (M < 16) return nblocks > 512;
   if (M <= 32 || (M <= 64 && N * K <= kSmallMWideElems)) return true;
-  const double tiles = (double)(((M + 127) / 128) * ((N + 127) / 128)) / (double)device_cus();
+  const int64_t cus = device_cus();
+  const double tiles = (double)(((M + 127) / 128) * ((N + 127) / 128)) / (double)cus;
   const double tiled = 3.5 + 0.45 * (double)kblocks * (tiles > 1.0 ? tiles : 1.0);
-  return 1.2 * midm_cost(midm_best(M, N, K), M, N, K) < tiled;
+  double cost = 0.0;
+  midm_best(M, N, K, cus, &cost);
+  return 1.2 * cost < tiled;
 }
 
 void midm_plan(int64_t M, int64_t N, int64_t K, int* fm, int* nb) {
@@ -236,7 +242,8 @@ void midm_plan(int64_t M, int64_t N, int64_t K, int* fm, int* nb) {
       *fm = s.fm, *nb = s.nb;
       return;
     }
-  const MidmSplit& s = midm_best(M, N, K);
+  double cost = 0.0;
+  const MidmSplit& s = midm_best(M, N, K, device_cus(), &cost);
   *fm = s.fm, *nb = s.nb;
 }
 
