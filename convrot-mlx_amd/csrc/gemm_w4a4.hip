@@ -2598,6 +2598,8 @@ constexpr Fp6Tile kFp6Tiles[5] = {{256, 256, 0.86}, {256, 224, 0.9}, {128, 256, 
 //   4608 x 3072 -> 12288, 96 over three:        114.6 | 109.3 | 115.1
 //   8192 x 3072 -> 3072, 128 over one:           68.0 |  63.2 |  69.2
 //   3072 x 3072 -> 9216, 176 over one:           60.2 |  70.0 |  71.7 (left as tiles)
+// and in four against the 128 x 128 tiles: 1536 x 3072 -> 12288 46.9 -> 43.0,
+// 4608 x 3072 -> 4096 55.7 -> 49.5.
 constexpr double kFp6Parts[2] = {0.58, 0.43};
 
 Fp6Tile fp6_tile(int64_t M, int64_t N, bool compact) {
