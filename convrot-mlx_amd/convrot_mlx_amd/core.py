@@ -894,15 +894,27 @@ def _linear_rows_eligible(x2d: torch.Tensor, group_size: int, a4: bool) -> bool:
             and rows * features * x2d.element_size() <= LINEAR_ROWS_MAX_BYTES)
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two contiguous tensors share a byte."""
+    pa, pb = a.data_ptr(), b.data_ptr()
+    return pa < pb + b.numel() * b.element_size() and pb < pa + a.numel() * a.element_size()
+
+
 def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, wscales, bias, n: int,
                  gr: GatedResidual | None) -> torch.Tensor:
-    """The whole layer on a few rows: `w` its CDNA4 weight, `gr` a residual that is not in place."""
+    """The whole layer on a few rows, `w` its CDNA4 weight.  In place, where the output may lie
+    over x (x its own residual), the launch reads a copy of x: every workgroup reads all of it."""
     m, k = x2d.shape
     _validate_mpp_epilogue(m, n, None, wscales, bias)
     device = nat.require_device(x2d, w, wscales, bias)
     x2d, w = x2d.contiguous(), w.contiguous()
     ws, b = _f32(wscales), _f32(bias)
-    out = torch.empty((m, n), dtype=x2d.dtype, device=device)
+    if gr is not None and gr.inplace:
+        out = gr.residual.view(m, n)
+        if _overlap(x2d, out):
+            x2d = x2d.clone()
+    else:
+        out = torch.empty((m, n), dtype=x2d.dtype, device=device)
     nat.check(
         nat.load().convrot_linear_rows(
             nat.ptr(x2d), nat.dtype_code(x2d.dtype), group_size, int(a4), nat.ptr(w), nat.ptr(ws), nat.ptr(b), m, n,
@@ -1098,18 +1110,19 @@ class ConvRotLinear(nn.Module):
         """linear(x); with `residual`, residual + gate * linear(x) (gate None: residual +
         linear(x)), each op rounded to x.dtype as torch evaluates it eagerly.  The gate
         broadcasts to the output ([B, 1, N] per image, [N], or full); `inplace` writes the
-        result into `residual` and returns it."""
+        result into `residual` and returns it, the same bits as out of place.  W4A4 sums are exact
+        integers; W4A16 sums are float32 in an order that the kernel of the row count has, so
+        rows of one batch need not have the bits they have alone."""
         if x.shape[-1] != self.in_features:
             raise ValueError(f"ConvRotLinear expected K={self.in_features}, got {x.shape[-1]}")
         x2d = x.reshape(-1, self.in_features)
-        # in place, the output may be x itself, which every workgroup of the one launch reads
-        if not inplace and (gate is None or residual is not None) and _linear_rows_eligible(x2d, self.group_size,
-                                                                                            self.a4):
+        if (residual is not None or (gate is None and not inplace)) and _linear_rows_eligible(x2d, self.group_size,
+                                                                                              self.a4):
             out_shape = (*x.shape[:-1], self.out_features)
             w = self._device_weight()
-            gr = None if residual is None else _gated_residual(residual, gate, out_shape, x.dtype)
-            return _linear_rows(x2d, self.group_size, self.a4, w, self.scales, self.bias, self.out_features,
-                                gr).reshape(out_shape)
+            gr = None if residual is None else _gated_residual(residual, gate, out_shape, x.dtype, inplace)
+            out = _linear_rows(x2d, self.group_size, self.a4, w, self.scales, self.bias, self.out_features, gr)
+            return residual if inplace else out.reshape(out_shape)
         return self._project(lambda mode: _prepare(x2d, self.group_size, mode), x.shape[:-1], x.dtype,
                              residual, gate, inplace)
 

@@ -134,3 +134,22 @@ def test_rows_nonfinite(orc, dev):
         assert torch.equal(got.nan_to_num(0.0)[0], want.nan_to_num(0.0)[0])
         if layer.a4:
             assert torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0))
+
+
+@pytest.mark.parametrize("backend", ["hip-w4a4", "hip-w4a16"])
+@pytest.mark.parametrize("M", [1, 3, 4, 8])
+def test_inplace_bits(orc, dev, backend, M):
+    """In place and out of place are the same bits: a residual of its own, x itself, and a residual that
+    starts inside x or in which x starts; x is read before any of it is written."""
+    K = N = 1024
+    layer, *_ = _layer(orc, dev, K, N, 256, backend, M)
+    gate = torch.randn(1, N, device=dev).bfloat16()
+    for offset in (None, 0, 8, N // 2 + 8, -8, -(N // 2)):  # elements from x's start to the residual's
+        for g in (None, gate):
+            buf = torch.randn(2 * M * N + N, device=dev).bfloat16()
+            x = buf[N // 2 :][: M * K].view(M, K)
+            start = N // 2 + offset if offset is not None else N // 2 + M * K
+            res = buf[start :][: M * N].view(M, N)
+            want = layer(x.clone(), residual=res.clone(), gate=g)
+            assert layer(x, residual=res, gate=g, inplace=True) is res
+            assert torch.equal(res, want), (offset, g is None)
