@@ -909,6 +909,9 @@ def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, 
     device = nat.require_device(x2d, w, wscales, bias)
     x2d, w = x2d.contiguous(), w.contiguous()
     ws, b = _f32(wscales), _f32(bias)
+    # not used here: a program that warms a stream up with a few rows and then captures
+    # more gets the plans that need the stream's workspace
+    _workspace(device)
     if gr is not None and gr.inplace:
         out = gr.residual.view(m, n)
         if _overlap(x2d, out):

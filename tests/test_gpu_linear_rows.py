@@ -153,3 +153,28 @@ def test_inplace_bits(orc, dev, backend, M):
             want = layer(x.clone(), residual=res.clone(), gate=g)
             assert layer(x, residual=res, gate=g, inplace=True) is res
             assert torch.equal(res, want), (offset, g is None)
+
+
+@pytest.mark.parametrize("backend", ["hip-w4a4", "hip-w4a16"])
+def test_few_rows_make_the_workspace(orc, dev, backend):
+    """A stream whose eager calls had one row has its workspace: a later capture of more rows runs the plan
+    (and, W4A16, the bits) of an eager call of those rows."""
+    from convrot_mlx_amd import core
+
+    layer, *_ = _layer(orc, dev, 12288, 512, 256, backend, 5)
+    x = torch.randn(32, 12288, device=dev).bfloat16()
+    want = layer(x)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    core._WORKSPACES.pop((stream.device.index, stream.cuda_stream), None)
+    with torch.cuda.stream(stream):
+        layer(x[:1])
+    torch.cuda.synchronize()
+    assert (stream.device.index, stream.cuda_stream) in core._WORKSPACES
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = layer(x)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
