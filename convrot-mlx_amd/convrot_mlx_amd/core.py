@@ -876,8 +876,10 @@ def hip_w4a16_matmul(activations, qweight, wscales, bias, *, output_dtype, out_f
 # W4A4 at K = 3072, M = 2: 6.5 -> 5.8 us (N = 3072), 12.8 -> 10.1 (18432); M = 3:
 # 6.55 -> 6.73, 13.1 -> 10.9; K = 1024 -> 1536, M = 4: 5.1 -> 4.8, M = 6: 5.1 -> 5.5.
 # W4A16 (no codes): K = 3072, M = 4: 7.2 -> 6.6, 13.5 -> 12.1; K = 1024, M = 8:
-# 6.0 -> 4.5; K = 8192, M = 2: 8.9 -> 9.3.  An eager call also saves ~8 us of host
-# work (a launch and two buffers).
+# 6.0 -> 4.5; K = 8192, M = 2: 8.9 -> 9.3.  An eager call also saves ~14 us of host
+# work (a launch and two buffers: 33.5 -> 19 us), which pays for the shapes inside the
+# bound that lose up to 0.6 us in a graph (K = 1536 -> 4096, G = 256: W4A4 M = 4
+# 6.19 -> 6.35, W4A16 M = 8 6.90 -> 7.54).
 LINEAR_ROWS_MAX = {True: (4, 6144), False: (8, 12288)}  # W4A4, W4A16: rows, elements of x
 LINEAR_ROWS_MAX_BYTES = 32768  # of x, include/convrot_amd.h
 LINEAR_ROWS_GROUPS = (64, 256)
@@ -909,9 +911,11 @@ def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, 
     device = nat.require_device(x2d, w, wscales, bias)
     x2d, w = x2d.contiguous(), w.contiguous()
     ws, b = _f32(wscales), _f32(bias)
+    stream = torch.cuda.current_stream(device).cuda_stream
     # not used here: a program that warms a stream up with a few rows and then captures
     # more gets the plans that need the stream's workspace
-    _workspace(device)
+    if (device.index, stream) not in _WORKSPACES:
+        _workspace(device)
     if gr is not None and gr.inplace:
         out = gr.residual.view(m, n)
         if _overlap(x2d, out):
@@ -923,7 +927,7 @@ def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, 
             nat.ptr(x2d), nat.dtype_code(x2d.dtype), group_size, int(a4), nat.ptr(w), nat.ptr(ws), nat.ptr(b), m, n,
             k, nat.ptr(gr.residual if gr is not None else None), nat.ptr(gr.gate if gr is not None else None),
             gr.stride if gr is not None else 0, gr.rows_per_gate if gr is not None else 1, nat.ptr(out),
-            nat.stream_of(device),
+            stream,
         )
     )
     return out
