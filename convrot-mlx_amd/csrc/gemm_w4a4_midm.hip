@@ -212,27 +212,32 @@ const MidmSplit& midm_best(int64_t M, int64_t N, int64_t K, int64_t cus, double*
 // weights once for every 16 rows (preparation and GEMM, HIP-graph replays, us:
 // M = 32, 3072 -> 9216 13.8 -> 8.8, 12288 -> 3072 15.1 -> 13.4; M = 16
 // 3072 -> 3072 7.5 -> 7.2), below that only where there are many weight tiles
-// (M = 6, 3072 -> 9216 9.1 -> 8.3, but 12288 -> 3072 10.9 -> 12.1 and M = 12,
-// 16384 -> 4096 16.3 -> 17.2).
+// (M = 6, 3072 -> 9216 9.1 -> 8.3, but 12288 -> 3072 10.9 -> 12.1, M = 12,
+// 16384 -> 4096 16.3 -> 17.2) and not too many (M = 5: 1024 -> 8448 6.4 -> 6.6,
+// 3072 -> 9216 8.8 -> 8.0, 16384 -> 12288 28.0 -> 27.1, 16384 -> 16384 30.7 -> 32.0).
 // Against the 128-row tiles, one of which walks K in ~0.47 us a k-block whatever
 // M, they win until their rounds add up: M = 77, 3072 -> 3072 19.9 -> 8.5,
 // 9216 19.9 -> 12.3, 12288 -> 3072 57.3 -> 17.8; M = 255, 3072 -> 3072
 // 20.4 -> 11.3, 12288 -> 3072 51.4 -> 26.4; but 3072 -> 18432 M = 64
-// 21.0 -> 16.9, M = 77 21.1 -> 24.4.  The model is 20 % low on many rounds.
+// 21.0 -> 16.9, M = 77 21.1 -> 24.4.  The model is 20 % low on many rounds, 40 %
+// where a wave has one or two k-blocks (1024 -> 18432, M = 77: 11.5 -> 12.0 if
+// taken) and 60 % on K past 12288 (16384 -> 16384, M = 77 56.8 -> 60.6, 16384 ->
+// 8448, M = 129 59.9 -> 62.0; but 12288 -> 12288, M = 129 56.9 -> 47.4).
 bool midm_preferred(int64_t M, int64_t N, int64_t K) {
   const int64_t nblocks = (N + 15) / 16, kblocks = (K + 127) / 128;
   if (M > 255 || M < 5 || N <= 0 || K <= 0) return false;
   if (tuning(kTuneMidmCfg) >= 0) return true;
   for (const TuneKey k : {kTuneGemmTile, kTuneGemmSk, kTuneGemmNoDma, kTuneGemmSmallmMax, kTuneW4a4SmallmCfg})
     if (tuning(k) >= 0) return false;  // a kernel of row-major codes is asked for
-  if (M < 16) return nblocks > 512;
+  if (M < 16) return nblocks > 512 && N * K < (1ll << 28);
   if (M <= 32 || (M <= 64 && N * K <= kSmallMWideElems)) return true;
   const int64_t cus = device_cus();
   const double tiles = (double)(((M + 127) / 128) * ((N + 127) / 128)) / (double)cus;
   const double tiled = 3.5 + 0.45 * (double)kblocks * (tiles > 1.0 ? tiles : 1.0);
   double cost = 0.0;
   midm_best(M, N, K, cus, &cost);
-  return 1.2 * cost < tiled;
+  const double low = kblocks < 16 ? 1.4 : kblocks > 96 ? 1.6 : 1.2;  // how far the model may be below
+  return low * cost < tiled;
 }
 
 void midm_plan(int64_t M, int64_t N, int64_t K, int* fm, int* nb) {

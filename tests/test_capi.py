@@ -322,3 +322,14 @@ def test_fp6_plan(lib, M, N, tile):
     bm, bn = ctypes.c_int(0), ctypes.c_int(0)
     assert lib.convrot_w4a4_fp6_tile(M, N, ctypes.byref(bm), ctypes.byref(bn)) == 0
     assert f"{bm.value}x{bn.value}" == tile
+
+
+# Where the W4A4 layer takes blocked codes, on 256 CUs: each side of the rule's lines.
+@pytest.mark.parametrize("M,N,K,takes", [
+    (77, 3072, 3072, 1), (255, 3072, 12288, 1), (129, 12288, 12288, 1), (129, 8448, 16384, 0), (65, 16384, 16384, 0),
+    (64, 16384, 16384, 1), (77, 18432, 1024, 0), (129, 8448, 1024, 1), (5, 8448, 1024, 1), (5, 8192, 1024, 0),
+    (5, 9216, 3072, 1), (5, 12288, 16384, 1), (5, 16384, 16384, 0), (16, 16384, 16384, 1),
+    (4, 9216, 3072, 0), (256, 3072, 3072, 0),
+])
+def test_blocked_rule(lib, M, N, K, takes):
+    assert lib.convrot_w4a4_blocked(M, N, K) == takes
