@@ -19,6 +19,7 @@ LIB_PATH = Path(__file__).resolve().parent / LIB_NAME
 DTYPE_F32, DTYPE_F16, DTYPE_BF16 = 0, 1, 2
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_LAUNCH = 0, 1, 2, 3
 PREP_PACKED, PREP_INT8, PREP_ROTATE, PREP_FP6, PREP_INT8_BLOCKED, PREP_NO_ROTATE = 0, 1, 2, 3, 4, 0x10
+PRODUCER_PLAIN, PRODUCER_MODULATE, PRODUCER_GELU = 0, 1, 2
 LAYOUT_NK, LAYOUT_KN, LAYOUT_CDNA4 = 0, 1, 2
 ACT_PACKED, ACT_INT8, ACT_INT8_BLOCKED = 0, 1, 2
 
@@ -29,6 +30,7 @@ SIGNATURES = {
     "convrot_prepare_modulated": (_i32, [_vp, _i32, _i64, _i64, _i32, _i32, _vp, _vp, _i64, ctypes.c_float, _vp,
                                          _vp, _vp]),
     "convrot_prepare_gelu": (_i32, [_vp, _i64, _i64, _vp, _i64, _i64, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
+    "convrot_prepare_plan": (_i32, [_i64, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
     "convrot_linear_rows": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _i64,
                                    _vp, _vp]),
     "convrot_w4a4_gemm": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i32, _vp]),
@@ -156,6 +158,15 @@ def cdna4_bytes(n: int, k: int) -> int:
 
 def fp6_bytes(rows: int, k: int) -> int:
     return int(load().convrot_fp6_bytes(rows, k))
+
+
+def prepare_plan(rows: int, features: int, dtype: int, group_size: int, mode: int,
+                 producer: int = PRODUCER_PLAIN) -> tuple[int, int, bool]:
+    """(1024-feature blocks a wave, waves a row, packed 16-bit kernel?) of a preparation."""
+    it, waves, packed = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+    check(load().convrot_prepare_plan(rows, features, dtype, group_size, mode, producer, ctypes.byref(it),
+                                      ctypes.byref(waves), ctypes.byref(packed)))
+    return it.value, waves.value, bool(packed.value)
 
 
 def fp6_tile(m: int, n: int) -> tuple[int, int]:

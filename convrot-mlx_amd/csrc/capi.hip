@@ -178,6 +178,21 @@ int convrot_w4a4_fp6_tile(int64_t M, int64_t N, int* bm, int* bn) {
   return ok();
 }
 
+int convrot_prepare_plan(int64_t rows, int64_t features, int dtype, int group_size, int mode, int producer,
+                         int* iterations, int* waves, int* packed) {
+  const bool no_rotate = (mode & CONVROT_PREP_NO_ROTATE) != 0;
+  const int kind = mode & ~CONVROT_PREP_NO_ROTATE, s = no_rotate ? 0 : log4_group(group_size);
+  if (rows < 0 || features <= 0 || features > kMaxFeatures || !valid_dtype(dtype) || s < 0 || s > 5 ||
+      kind < CONVROT_PREP_PACKED || kind > CONVROT_PREP_INT8_BLOCKED || producer < CONVROT_PRODUCER_PLAIN ||
+      producer > CONVROT_PRODUCER_GELU || !iterations || !waves || !packed)
+    return fail(CONVROT_ERR_INVALID, "preparation plan query: bad shape, dtype, group, mode, producer or result pointer");
+  bool p = false;
+  if (!convrot::prep_route(rows, features, dtype, s, kind, producer, iterations, waves, &p))
+    return fail(CONVROT_ERR_UNSUPPORTED, "no preparation plan for %lld features", (long long)features);
+  *packed = p ? 1 : 0;
+  return ok();
+}
+
 int convrot_prepare(const void* x, int dtype, int64_t rows, int64_t features, int group_size, int mode,
                     void* out, float* scales, void* stream) {
   const bool no_rotate = (mode & CONVROT_PREP_NO_ROTATE) != 0;

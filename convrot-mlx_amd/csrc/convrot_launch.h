@@ -46,7 +46,11 @@ bool w4a16_tile_known(int bm, int bn);
 // blocks; compact weights may split the last round of a 256 x 256 grid instead.
 void fp6_plan_tile(int64_t M, int64_t N, int* bm, int* bn);
 
-bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out, bool packed);
+// What the preparation of such rows runs: iterations a wave, waves a row, and
+// whether on the kernel of packed 16-bit values (the CONVROT_PRODUCER_* codes).
+// False: no split covers the features.
+bool prep_route(int64_t rows, int64_t K, int dtype, int log4g, int mode, int producer, int* iterations, int* waves,
+                bool* packed);
 
 hipError_t launch_prep(const void* x, int dtype, int64_t rows, int64_t K, int log4g, int mode, void* out,
                        float* scales, hipStream_t stream);

@@ -146,9 +146,9 @@ __device__ __forceinline__ float gelu_tanh32(float x) {
 
 // Producers: what the preparation reads as its input rows.
 enum Producer : int {
-  kProPlain = 0,     // x
-  kProModulate = 1,  // (1 + scale) * layer_norm(x) + shift
-  kProGelu = 2,      // [head | gelu_tanh(x)], each with its own row stride
+  kProPlain = CONVROT_PRODUCER_PLAIN,        // x
+  kProModulate = CONVROT_PRODUCER_MODULATE,  // (1 + scale) * layer_norm(x) + shift
+  kProGelu = CONVROT_PRODUCER_GELU,          // [head | gelu_tanh(x)], each with its own row stride
 };
 
 // Arguments of the producers beyond x (unused fields are ignored).
@@ -966,9 +966,46 @@ void prep16_kernel(const void* __restrict__ x, void* __restrict__ out,
   }
 }
 
-// Whether prep16_kernel prepares these rows.
-constexpr bool prep_packed(int dtype, int log4g, int mode) {
-  return log4g >= 1 && (dtype == kF16 || (dtype == kBF16 && mode != CONVROT_PREP_ROTATE));
+// Which rows prep16_kernel prepares; rounding and codes are the same on both.
+// prep_kernel stays the faster one (us, prep16_kernel against it) for
+//  * bf16 rows of four blocks a wave behind the modulated producer, which spill
+//    (8800 x 16384: 193 against 174);
+//  * plain bf16 rows of groups up to 64 with FP6 output up to 16384 features, where
+//    the butterfly is short and the FP6 stores are the bound: finishing rows sooner,
+//    prep16_kernel has more 16-row blocks open at once and writes their lines back
+//    in more pieces (8800 x 16384, G = 64: 118-123 MB against 108, 104 against
+//    96; 4877 x 29568, many more waves a row: 110 against 149).  G = 64 wins up to
+//    12288 features and on few rows (1536 x 16384: 22.2 against 30.8); G = 16 only
+//    on very short rows or few 1024-feature blocks in all (8800 x 8192 57 against 55,
+//    2000 x 12288 22.5 against 19.7, but 7020 x 1152 9.4 against 10.2, 381 x 12288
+//    7.0 against 7.2);
+//  * other plain bf16 rows of groups of 4, there (packed 1061 x 14336 13.5 against
+//    12.4; int8 682 x 28032 17.2 against 18.0);
+//  * float16 ROTATE on one iteration: plain at G = 64 beyond 10240 features and
+//    12288 blocks in all (2000 x 12288 22.3 against 21.2; 2048 x 10240 19.7 against
+//    20.1, 710 x 14336 11.4 against 12.2), modulated at G up to 16 (5879 x 7168,
+//    G = 16: 43.5 against 40.3).
+enum Packed : int { kNoRows, kCode64Rows, kCode16Rows, kRotateRows, kAllRows };
+constexpr int64_t kFewRows = 2048, kFewBlocks = 12288;
+constexpr Packed prep_packed(int dtype, int log4g, int ni, int mode, int producer) {
+  if (log4g < 1 || dtype == kF32) return kNoRows;
+  if (dtype == kBF16) {
+    if (mode == CONVROT_PREP_ROTATE || (producer == kProModulate && ni == 4)) return kNoRows;
+    if (producer == kProPlain && (log4g == 1 || (mode == CONVROT_PREP_FP6 && log4g <= 3)))
+      return log4g == 3 ? kCode64Rows : kCode16Rows;
+  } else if (mode == CONVROT_PREP_ROTATE && ni == 1) {
+    if (producer == kProPlain && log4g == 3) return kRotateRows;
+    if (producer == kProModulate && log4g <= 2) return kNoRows;
+  }
+  return kAllRows;
+}
+constexpr bool prep_packed_rows(Packed p, int64_t rows, int64_t K) {
+  switch (p) {
+    case kCode64Rows: return K <= 12288 || K > 16384 || rows <= kFewRows;
+    case kCode16Rows: return K < 2048 || K > 16384 || rows * ((K + 1023) / 1024) < kFewBlocks;
+    case kRotateRows: return K <= 10240 || rows * ((K + 1023) / 1024) < kFewBlocks;
+    default: return p == kAllRows;
+  }
 }
 
 // The producer of a launch and its arguments.
@@ -977,31 +1014,32 @@ struct Modulation {
   ProducerArgs args;
 };
 
+template <int DT, int S, int NI, int MODE, int PRO>
+void launch_prep_pro(const void* x, void* out, float* scales, int64_t rows, int K, int waves, const ProducerArgs& args,
+                     hipStream_t stream) {
+  constexpr Packed kPacked = prep_packed(DT, S, NI, MODE, PRO);
+  const auto launch = [&](void (*kernel)(const void*, void*, float*, int, ProducerArgs), int region) {
+    const size_t lds_bytes = S >= 3 ? (size_t)waves * (size_t)region * 4 : 0;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(64 * waves), lds_bytes, stream, x, out, scales, K, args);
+  };
+  if constexpr (kPacked != kNoRows) {
+    if (prep_packed_rows(kPacked, rows, K)) return launch(prep16_kernel<DT, S, NI, MODE, PRO>, kPkRegion);
+  }
+  if constexpr (kPacked != kAllRows) launch(prep_kernel<DT, S, NI, MODE, PRO>, kRegionFloats);
+}
+
 template <int DT, int S, int NI, int MODE>
 hipError_t launch_prep_t(const void* x, void* out, float* scales, int64_t rows, int K, int waves,
                          const Modulation& mod, hipStream_t stream) {
-  constexpr bool kPacked = prep_packed(DT, S, MODE);
-  const auto launch = [&](void (*kernel)(const void*, void*, float*, int, ProducerArgs), int region) {
-    const size_t lds_bytes = S >= 3 ? (size_t)waves * (size_t)region * 4 : 0;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(64 * waves), lds_bytes, stream, x, out, scales, K, mod.args);
-  };
-  if constexpr (kPacked) {
-    // bf16 rows of four blocks a wave behind the modulated producer spill on the packed kernel (8800 x 16384:
-    // 193 us against 174 on the other)
-    if (mod.producer == kProModulate) {
-      if constexpr (DT == kBF16 && NI == 4) launch(prep_kernel<DT, S, NI, MODE, kProModulate>, kRegionFloats);
-      else launch(prep16_kernel<DT, S, NI, MODE, kProModulate>, kPkRegion);
-    } else if (mod.producer == kProGelu) {
-      launch(prep16_kernel<DT, S, NI, MODE, kProGelu>, kPkRegion);
-    } else {
-      launch(prep16_kernel<DT, S, NI, MODE, kProPlain>, kPkRegion);
-    }
-  } else if constexpr (S == 0) {  // no rotation: the plain producer only
-    launch(prep_kernel<DT, S, NI, MODE, kProPlain>, kRegionFloats);
+  if constexpr (S == 0) {  // no rotation: the plain producer only
+    launch_prep_pro<DT, S, NI, MODE, kProPlain>(x, out, scales, rows, K, waves, mod.args, stream);
   } else {
-    if (mod.producer == kProModulate) launch(prep_kernel<DT, S, NI, MODE, kProModulate>, kRegionFloats);
-    else if (mod.producer == kProGelu) launch(prep_kernel<DT, S, NI, MODE, kProGelu>, kRegionFloats);
-    else launch(prep_kernel<DT, S, NI, MODE, kProPlain>, kRegionFloats);
+    if (mod.producer == kProModulate)
+      launch_prep_pro<DT, S, NI, MODE, kProModulate>(x, out, scales, rows, K, waves, mod.args, stream);
+    else if (mod.producer == kProGelu)
+      launch_prep_pro<DT, S, NI, MODE, kProGelu>(x, out, scales, rows, K, waves, mod.args, stream);
+    else
+      launch_prep_pro<DT, S, NI, MODE, kProPlain>(x, out, scales, rows, K, waves, mod.args, stream);
   }
   return hipGetLastError();
 }
@@ -1050,11 +1088,20 @@ hipError_t launch_prep_s(int s, int ni, int mode, const void* x, void* out, floa
 // Pick (iterations per wave, waves per row) so that 1024*NI*W covers K with
 // the fewest idle 1024-feature blocks; NI in {3, 4, 1}, W <= 16.  Few rows
 // (M <= 2048) take one iteration per wave and more waves per row instead, so
-// that enough waves are in flight to cover the load latency; the packed kernel
-// only up to 12288 blocks in all (1536 x 15360, one iteration -> four: 21.4 ->
-// 18.7 us, modulated 39.1 -> 34.2; the other kernel and the GELU producer gain
-// nothing there: `packed` is false for them).
-bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out, bool packed) {
+// that enough waves are in flight to cover the load latency.  The packed kernel
+// differs (us):
+//  * few rows take one iteration only up to 12288 blocks in all (bf16 1536 x 15360,
+//    one -> four: 21.4 -> 18.7, modulated 39.1 -> 34.2, though that runs on
+//    prep_kernel, and not on two waves: 1667 x 8192 21.5 -> 25.3).  Plain rotated
+//    outputs (float16 2000 x 12288, G = 64: 22.5 -> 24.9), the GELU producer and plain
+//    groups up to 16 of at most 12 blocks (bf16 1536 x 12288, G = 16: 12.5 -> 13.6)
+//    gain nothing;
+//  * plain FP6 rows of groups up to 64 (bf16: 64, up to 12288 features) take one
+//    iteration where four would be taken, with fewer rows and so fewer 16-row blocks
+//    open: bf16 G = 64 8800 x 8192 58.3 -> 51.4, float16 G = 16 8800 x 16384 124 -> 93.5;
+//  * else 13 to 16 blocks are four waves of four, as 15 and 16 are on any kernel
+//    (bf16 G = 256 FP6 4608 x 13312, thirteen of one -> four of four: 58.0 -> 47.8).
+static bool prep_plan(int64_t rows, int64_t K, int dtype, int log4g, int mode, int producer, int* ni_out, int* waves_out) {
   const int64_t blocks = (K + 1023) / 1024;
   {  // tuning override: force the iterations per wave
     const int ni = tuning(kTunePrepNi);
@@ -1067,9 +1114,21 @@ bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out, bool packed
       }
     }
   }
-  if (rows <= 2048 && blocks <= kMaxWaves && !(packed && rows * blocks > 12288)) {
+  const Packed packed = prep_packed(dtype, log4g, 3, mode, producer);
+  const bool coded = packed != kNoRows && packed != kCode16Rows && producer != kProGelu &&
+                     !(producer == kProPlain && mode == CONVROT_PREP_ROTATE);
+  const bool deep = coded && rows * blocks > kFewBlocks && (log4g > 2 || producer != kProPlain || blocks > 12) &&
+                    (dtype != kBF16 || producer != kProModulate || blocks > 8);
+  const bool spread = producer == kProPlain && mode == CONVROT_PREP_FP6 &&
+                      (packed == kCode64Rows ? K <= 12288 : packed == kAllRows && log4g <= 2);
+  if (blocks <= kMaxWaves && rows <= kFewRows && !deep) {
     *ni_out = 1;
     *waves_out = (int)blocks;
+    return true;
+  }
+  if (coded && blocks > 12 && blocks <= 16) {
+    *ni_out = spread ? 1 : 4;
+    *waves_out = spread ? (int)blocks : 4;
     return true;
   }
   int best_ni = 0, best_w = 0;
@@ -1098,8 +1157,16 @@ bool prep_plan(int64_t rows, int64_t K, int* ni_out, int* waves_out, bool packed
     }
   }
   if (best_idle < 0) return false;
+  if (spread && best_ni == 4 && blocks <= kMaxWaves) best_ni = 1, best_w = (int)blocks;
   *ni_out = best_ni;
   *waves_out = best_w;
+  return true;
+}
+
+bool prep_route(int64_t rows, int64_t K, int dtype, int log4g, int mode, int producer, int* iterations, int* waves,
+                bool* packed) {
+  if (!prep_plan(rows, K, dtype, log4g, mode, producer, iterations, waves)) return false;
+  *packed = prep_packed_rows(prep_packed(dtype, log4g, *iterations, mode, producer), rows, K);
   return true;
 }
 
@@ -1108,7 +1175,7 @@ namespace {
 hipError_t launch_prep_any(const void* x, int dtype, int64_t rows, int64_t K, int log4g, int mode, void* out,
                            float* scales, const Modulation& mod, hipStream_t stream) {
   int ni = 0, waves = 0;
-  if (!prep_plan(rows, K, &ni, &waves, prep_packed(dtype, log4g, mode) && mod.producer != kProGelu)) return hipErrorInvalidValue;
+  if (!prep_plan(rows, K, dtype, log4g, mode, mod.producer, &ni, &waves)) return hipErrorInvalidValue;
   if (rows == 0) return hipSuccess;
   switch (dtype) {
     case kF32: return launch_prep_s<kF32>(log4g, ni, mode, x, out, scales, rows, (int)K, waves, mod, stream);

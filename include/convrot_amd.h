@@ -60,6 +60,10 @@ extern "C" {
 #define CONVROT_PREP_INT8_BLOCKED 4 /* out: int8 A4 codes in [ceil(features/128)][ceil(rows/16)][2048] blocks, + scales:
                                * feature f = 32 q + 16 s + b (q 0..3, s 0..1, b 0..15) of the block's row r at
                                * byte 1024 s + 16 (16 q + r) + b; rows and features past the end are not written */
+/* producers of the prepared rows (convrot_prepare, convrot_prepare_modulated, convrot_prepare_gelu) */
+#define CONVROT_PRODUCER_PLAIN 0
+#define CONVROT_PRODUCER_MODULATE 1
+#define CONVROT_PRODUCER_GELU 2
 /* OR-able flag: skip the rotation (quantize_signed_int4_rowwise semantics) */
 #define CONVROT_PREP_NO_ROTATE 0x10
 
@@ -128,6 +132,15 @@ int convrot_prepare_modulated(const void* x, int dtype, int64_t rows, int64_t fe
 int convrot_prepare_gelu(const void* head, int64_t head_features, int64_t head_stride, const void* x,
                          int64_t x_features, int64_t x_stride, int dtype, int64_t rows, int group_size, int mode,
                          void* out, float* scales, void* stream);
+
+/*
+ * What a preparation of such rows runs: 1024-feature blocks a wave, waves a row,
+ * and whether on the kernel of packed 16-bit values (1) or of float32 values (0).
+ * The outputs are the same bits.  An introspection call for sweeps and tests,
+ * like convrot_w4a4_fp6_tile; no counterpart in the reference.
+ */
+int convrot_prepare_plan(int64_t rows, int64_t features, int dtype, int group_size, int mode, int producer,
+                         int* iterations, int* waves, int* packed);
 
 /*
  * The ConvRot linear of a few rows in one launch, from x to the output:

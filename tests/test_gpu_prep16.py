@@ -110,3 +110,34 @@ def test_gelu_every_value(orc, dev, dtype):
     codes, scales = orc.prepare_codes(x16, dtype, 64)
     got, s = core._prepare_gelu(to_dev(bits, dtype, dev), to_dev(head, dtype, dev), 64, nat.PREP_PACKED)
     assert np.array_equal(from_dev(got), orc.pack_signed_int4(codes)) and np.array_equal(from_dev(s), scales)
+
+
+@pytest.mark.parametrize("dtype,G,M,K,mode,cut", [("bfloat16", 64, 2080, 13312, "fp6", 1040),
+                                                  ("bfloat16", 64, 2080, 8192, "fp6", 1040),
+                                                  ("bfloat16", 16, 1600, 8192, "fp6", 800),
+                                                  ("float16", 16, 2080, 16384, "fp6", 1040),
+                                                  ("float16", 64, 2000, 12288, "rotate", 1000)])
+def test_routes_agree(dev, tuning, dtype, G, M, K, mode, cut):
+    """The automatic kernel and split of all the rows, and those of a part of them with every number of
+    iterations: other routes, the same bytes."""
+    from convrot_mlx_amd import _native as nat
+    from convrot_mlx_amd import core
+
+    dt = {"bfloat16": torch.bfloat16, "float16": torch.float16}[dtype]
+    kind = {"fp6": nat.PREP_FP6, "rotate": nat.PREP_ROTATE}[mode]
+    plan = lambda m: nat.prepare_plan(m, K, nat.dtype_code(dt), G, kind)  # noqa: E731
+    x = (torch.randn(M, K, device=dev) * 3).to(dt)
+    route = plan(M)
+    whole, s = core._prepare(x, G, kind)
+    others = set()
+    for ni in (None, 1, 3, 4):
+        tuning.set("prep_ni", ni)
+        others.add(plan(cut))
+        for i in range(0, M, cut):
+            part, sp = core._prepare(x[i : i + cut], G, kind)
+            if mode == "rotate":
+                assert torch.equal(whole[i : i + cut].view(torch.int16), part.view(torch.int16))
+            else:
+                assert torch.equal(whole[:, i // 16 : (i + cut) // 16], part) and torch.equal(s[i : i + cut], sp)
+    tuning.set("prep_ni", None)
+    assert len(others - {route}) >= 2
