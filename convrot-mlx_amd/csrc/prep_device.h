@@ -1,7 +1,8 @@
 // Device pieces of the ConvRot preparation shared by the preparation kernel
 // (prep.hip) and the few-row linear (linear_rows.hip): the butterfly with its
 // per-op rounding, the lane <-> feature layout of a wave's 1024-feature block
-// and its LDS exchanges, row loads, the row scale and the code of a ratio.
+// and its LDS exchanges, row loads, the row scale, the code of a ratio and the
+// GELU producer's tanh GELU.
 // The layout is described in prep.hip.
 #pragma once
 
@@ -210,6 +211,53 @@ template <int DT>
 __device__ __forceinline__ float code_ratio(float v, const RowScale<DT>& s) {
   if constexpr (DT == kBF16) return round_bf16(v * s.inv);
   else return s.scale > 0.0f ? rnd<DT>(v / s.scale) : 0.0f;  // 0/0 on an all-zero f16 row
+}
+
+// 1 / d, correctly rounded, for d in [1, 2^126): one Newton step from v_rcp_f32.
+// The step alone would leave a start value one ulp below at the all-ones
+// significand wrong; the hardware's is not.  Every float32 of the range is
+// compared with the float64 quotient in tests/test_gpu_device_checks.py.
+__device__ __forceinline__ float rcp_newton(float d) {
+  const float y = __builtin_amdgcn_rcpf(d);
+  return __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+}
+
+// tanh GELU of the fused GELU producer, float32, in this fixed sequence (the
+// same IEEE operations, in the same order, as the CPU oracle's gelu_tanh32):
+//   x3 = (x * x) * x;  u = kBeta * fma(kKappa, x3, x)
+//   q = 2 / (exp(2|u|) + 1)  (0 where 2|u| > 88 or u is NaN)
+//   1 + tanh(u) = u >= 0 ? 2 - q : q  (no cancellation on either side)
+//   y = (0.5 * x) * (1 + tanh(u))
+// with exp(z) = 2^n e^r, n = rint(z log2 e), r = z - n ln2 by two fmas
+// (Cody-Waite), e^r by its degree-7 Taylor polynomial (Horner, fma).
+//
+// Cheaper forms of the same values:
+//  * rint by adding and subtracting 1.5 * 2^23 (|z log2 e| < 2^7), which leaves
+//    n in the low bits of the sum: 2^n p is an integer add to p's exponent
+//    (p in [0.7, 1.42], n <= 127: no overflow, no denormal);
+//  * 2 / s as the reciprocal of s / 2 (exact halving), by rcp_newton.
+// 35 VALU operations with a conversion and a division in them became 29.
+__device__ __forceinline__ float gelu_tanh32(float x) {
+  const float x3 = (x * x) * x;
+  const float u = 0x1.988454p-1f * __builtin_fmaf(0x1.6e4e26p-5f, x3, x);
+  const float z = fabsf(u) + fabsf(u);
+  const float t = z * 0x1.715476p+0f + 12582912.0f;
+  const float n = t - 12582912.0f;
+  float r = __builtin_fmaf(-n, 0x1.62e4p-1f, z);
+  r = __builtin_fmaf(-n, 0x1.7f7d1cp-20f, r);
+  float p = 0x1.a01a02p-13f;
+  p = __builtin_fmaf(p, r, 0x1.6c16c2p-10f);
+  p = __builtin_fmaf(p, r, 0x1.111112p-7f);
+  p = __builtin_fmaf(p, r, 0x1.555556p-5f);
+  p = __builtin_fmaf(p, r, 0x1.555556p-3f);
+  p = __builtin_fmaf(p, r, 0x1p-1f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  const float e = __uint_as_float(__float_as_uint(p) + (__float_as_uint(t) << 23));
+  const float d = 0.5f * (e + 1.0f);
+  const float q = z <= 88.0f ? rcp_newton(d) : 0.0f;
+  const float onept = u >= 0.0f ? 2.0f - q : q;
+  return (0.5f * x) * onept;
 }
 
 }  // namespace convrot
