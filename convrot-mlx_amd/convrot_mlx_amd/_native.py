@@ -54,6 +54,7 @@ SIGNATURES = {
     "convrot_fp6_bytes": (_i64, [_i64, _i64]),
     "convrot_w4a4_blocked": (_i32, [_i64, _i64, _i64]),
     "convrot_w4a4_fp6_tile": (_i32, [_i64, _i64, _vp, _vp]),
+    "convrot_w4a4_fp6_compact_tile": (_i32, [_i64, _i64, _vp, _vp, _vp]),
     "convrot_weight_fp6": (_i32, [_vp, _vp, _i64, _i64, _vp]),
     "convrot_w4a4_gemm_fp6": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i32, _vp]),
     "convrot_w4a4_gemm_fp6_residual": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _i64, _vp,
@@ -174,3 +175,11 @@ def fp6_tile(m: int, n: int) -> tuple[int, int]:
     bm, bn = ctypes.c_int(0), ctypes.c_int(0)
     check(load().convrot_w4a4_fp6_tile(m, n, ctypes.byref(bm), ctypes.byref(bn)))
     return bm.value, bn.value
+
+
+def fp6_compact_tile(m: int, n: int) -> tuple[int, int, int]:
+    """The (BM, BN) tile of an m x n product on compact FP6 weights, and the workgroups that each tile
+    past the whole rounds runs as."""
+    bm, bn, parts = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+    check(load().convrot_w4a4_fp6_compact_tile(m, n, ctypes.byref(bm), ctypes.byref(bn), ctypes.byref(parts)))
+    return bm.value, bn.value, parts.value

@@ -178,6 +178,13 @@ int convrot_w4a4_fp6_tile(int64_t M, int64_t N, int* bm, int* bn) {
   return ok();
 }
 
+int convrot_w4a4_fp6_compact_tile(int64_t M, int64_t N, int* bm, int* bn, int* parts) {
+  if (M <= 0 || N <= 0 || !bm || !bn || !parts)
+    return fail(CONVROT_ERR_INVALID, "compact FP6 tile query needs M, N > 0 and three result pointers");
+  convrot::fp6_plan_compact(M, N, bm, bn, parts);
+  return ok();
+}
+
 int convrot_prepare_plan(int64_t rows, int64_t features, int dtype, int group_size, int mode, int producer,
                          int* iterations, int* waves, int* packed) {
   const bool no_rotate = (mode & CONVROT_PREP_NO_ROTATE) != 0;

@@ -43,8 +43,10 @@ bool fp6_tile_known(int bm, int bn);
 bool w4a16_tile_known(int bm, int bn);
 
 // The FP6 W4A4 tile the plan (and the fp6_tile override) picks for M x N on operand
-// blocks; compact weights may split the last round of a 256 x 256 grid instead.
+// blocks, and on compact weights, where each 256 x 256 tile past the whole rounds
+// may run as `parts` (1, 2 or 4) workgroups.
 void fp6_plan_tile(int64_t M, int64_t N, int* bm, int* bn);
+void fp6_plan_compact(int64_t M, int64_t N, int* bm, int* bn, int* parts);
 
 // What the preparation of such rows runs: iterations a wave, waves a row, and
 // whether on the kernel of packed 16-bit values (the CONVROT_PRODUCER_* codes).

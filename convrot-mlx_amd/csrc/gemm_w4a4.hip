@@ -2707,6 +2707,13 @@ void fp6_plan_tile(int64_t M, int64_t N, int* bm, int* bn) {
   *bn = t.bn;
 }
 
+void fp6_plan_compact(int64_t M, int64_t N, int* bm, int* bn, int* parts) {
+  const Fp6Tile t = fp6_tile(M, N, true);
+  *bm = t.bm;
+  *bn = t.bn;
+  *parts = t.sub;
+}
+
 hipError_t launch_w4a4_gemm_fp6(const uint8_t* act6, const float* xscales, const uint8_t* w6, const float* wscales,
                                 const float* bias, int64_t M, int64_t N, int64_t K, void* out, int out_dtype,
                                 hipStream_t stream, const GatedResidual& gr, bool compact_weights) {

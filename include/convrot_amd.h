@@ -355,10 +355,12 @@ int64_t convrot_fp6_bytes(int64_t R, int64_t K);
  * The BM x BN tile convrot_w4a4_gemm_fp6 runs for an M x N product (the
  * automatic plan, or the fp6_tile tuning override): an introspection call for
  * sweeps and tests, no counterpart in the reference.
- * convrot_w4a4_gemm_fp6_compact runs the same tile, or a 256 x 256 grid whose
- * last partial round is split into smaller workgroups (the same bits).
+ * convrot_w4a4_gemm_fp6_compact runs the tile of convrot_w4a4_fp6_compact_tile:
+ * the same one, or a 256 x 256 grid whose last partial round runs each tile as
+ * *parts = 2 or 4 workgroups (else 1; the same bits).
  */
 int convrot_w4a4_fp6_tile(int64_t M, int64_t N, int* bm, int* bn);
+int convrot_w4a4_fp6_compact_tile(int64_t M, int64_t N, int* bm, int* bn, int* parts);
 
 /*
  * CDNA4-layout weight -> FP6 operand blocks (an offline conversion, like

@@ -333,3 +333,40 @@ def test_fp6_plan(lib, M, N, tile):
 ])
 def test_blocked_rule(lib, M, N, K, takes):
     assert lib.convrot_w4a4_blocked(M, N, K) == takes
+
+
+# On compact weights, the layer's form: the leftover tiles of the last round (the comment's count) and the
+# workgroups each of them runs as.  Up to 64 leftover tiles go in four, up to 128 in two, more stay whole.
+@pytest.mark.parametrize("M,N,tile,parts", [
+    (8800, 4096, "256x256", 4),    # 48 over two rounds
+    (4608, 3840, "256x256", 4),    # 14 over one
+    (6144, 6144, "256x256", 4),    # 64 over two
+    (1536, 12288, "256x256", 4),   # 32 over one (128x128 tiles on operand blocks)
+    (2304, 9216, "256x256", 2),    # 68 over one
+    (4608, 12288, "256x256", 2),   # 96 over three
+    (8192, 3072, "256x256", 2),    # 128 over one
+    (8448, 3072, "256x256", 1),    # 140 over one
+    (3072, 9216, "256x256", 1),    # 176 over one
+    (10017, 2688, "256x256", 1),   # 184 over one
+    (4608, 3072, "256x256", 1),    # 216, less than a round
+    (4096, 4096, "256x256", 1),    # 256, a whole round
+    (1536, 3072, "128x192", 1), (512, 3072, "128x128", 1),
+])
+def test_fp6_compact_plan(lib, M, N, tile, parts):
+    from convrot_mlx_amd import _native as nat
+
+    bm, bn, got = nat.fp6_compact_tile(M, N)
+    assert (f"{bm}x{bn}", got) == (tile, parts)
+    assert lib.convrot_w4a4_fp6_compact_tile(M, 0, None, None, None) == 1
+
+
+@pytest.mark.parametrize("name,value,want", [("fp6_split", "1", (256, 256, 1)), ("fp6_split", "2", (256, 256, 2)),
+                                             ("fp6_tile", "128x256", (128, 256, 1))])
+def test_fp6_compact_plan_overrides(lib, name, value, want):
+    from convrot_mlx_amd import _native as nat
+
+    try:
+        nat.set_tuning(name, value)
+        assert nat.fp6_compact_tile(8800, 4096) == want
+    finally:
+        nat.set_tuning(name, None)
