@@ -242,8 +242,7 @@ hipError_t launch_rows_t(const void* x, const uint8_t* wq, const float* ws, cons
   const int nblocks = (int)((N + 15) / 16), kblocks = (int)((K + 127) / 128);
   const int groups = (nblocks + TG - 1) / TG;
   const RowsLds lay = rows_lds(M, kblocks, DT == kF32 ? 4 : 2, A4, TG * KS);
-  const int slots = (TG * KS <= 8 && lay.bytes <= 80 * 1024 - 256 ? 2 : 1) * device_cus();
-  hipLaunchKernelGGL((linear_rows_kernel<DT, S, A4, TG, KS, KPW>), dim3((unsigned)std::min(groups, slots)),
+  hipLaunchKernelGGL((linear_rows_kernel<DT, S, A4, TG, KS, KPW>), dim3((unsigned)std::min(groups, device_cus())),
                      dim3(64 * TG * KS), (size_t)lay.bytes, stream, x, wq, ws, bias, out, (int)M, (int)N, (int)K,
                      nblocks, kblocks, groups, lay, gr);
   return hipGetLastError();
@@ -282,10 +281,10 @@ int rows_split(int64_t N, int64_t K) {
   int64_t best_cost = INT64_MAX;
   for (const RowsSplit& c : kRowsSplits) {
     const int64_t groups = (nblocks + c.tg - 1) / c.tg;
-    const int64_t per_cu = c.cfg == 1 && groups > cus ? 2 : 1;  // two workgroups of eight waves share a CU
-    const int64_t rounds = (groups + cus * per_cu - 1) / (cus * per_cu);
+    if (c.cfg == 1 && groups > cus) continue;  // two tiles a workgroup load as much in fewer rounds
+    const int64_t rounds = (groups + cus - 1) / cus;
     const int64_t batches = (kblocks + c.ks * c.kpw - 1) / (c.ks * c.kpw);
-    const int64_t cost = rounds * (batches * per_cu * c.tg * c.ks * c.kpw + 24);
+    const int64_t cost = rounds * (batches * c.tg * c.ks * c.kpw + 24);
     // one tile a workgroup: sixteen waves where they tie on a long K (8192 -> 2048: 7.03 against 7.14)
     if (cost < best_cost || (cost == best_cost && c.cfg == 16 && K > 6144)) best = c.cfg, best_cost = cost;
   }
