@@ -252,8 +252,8 @@ hipError_t launch_rows_t(const void* x, const uint8_t* wq, const float* ws, cons
 //   rounds of workgroups over the CUs x (k-blocks a CU loads in a round + 24),
 // the loaded blocks counted whole batches of KS * KPW, and 24 for what a round
 // costs besides: as many tiles a workgroup as make one round (a CU prepares the
-// rows once), but no batch that is mostly past K.  It is within 1.6 % of the
-// best of the five at each of 27 shapes timed but one (5 %).  Measured at M = 1,
+// rows once), but no batch that is mostly past K.  At M = 1 it is within 1.6 % of
+// the best of the five at each of 27 shapes timed but one (5 %).  Measured at M = 1,
 // bf16, the preparation and GEMM launches against this one (HIP-graph replays
 // over > 256 MB of weights, us):
 //   K -> N         W4A4             W4A16            tiles, (TG, KS, KPW)
@@ -274,7 +274,7 @@ struct RowsSplit {
 };
 constexpr RowsSplit kRowsSplits[] = {{5, 5, 3, 8}, {3, 3, 5, 5}, {2, 2, 8, 3}, {1, 1, 8, 3}, {16, 1, 16, 3}};
 
-int rows_split(int64_t N, int64_t K) {
+int rows_split(int64_t N, int64_t K, bool a4) {
   if (const int v = tuning(kTuneRowsCfg); v >= 0) return v;
   const int64_t nblocks = (N + 15) / 16, kblocks = (K + 127) / 128, cus = device_cus();
   int best = 1;
@@ -285,8 +285,12 @@ int rows_split(int64_t N, int64_t K) {
     const int64_t rounds = (groups + cus - 1) / cus;
     const int64_t batches = (kblocks + c.ks * c.kpw - 1) / (c.ks * c.kpw);
     const int64_t cost = rounds * (batches * c.tg * c.ks * c.kpw + 24);
-    // one tile a workgroup: sixteen waves where they tie on a long K (8192 -> 2048: 7.03 against 7.14)
-    if (cost < best_cost || (cost == best_cost && c.cfg == 16 && K > 6144)) best = c.cfg, best_cost = cost;
+    // ties: one tile a workgroup, sixteen waves on a long K (8192 -> 2048: 7.03 against 7.14); W4A16 of 769
+    // to 1024 tiles, two rounds of two tiles on sixteen waves instead of one of five on fifteen, to expand the
+    // weights (3072 -> 14336, M = 1 9.66 against 9.89, M = 3 10.5 against 11.1; 2304 -> 14336 9.66 against 9.48)
+    const bool wide = c.cfg == 2 && best == 5 && !a4 && K >= 2560 && nblocks <= 4 * cus;
+    const bool tie = cost == best_cost && ((c.cfg == 16 && K > 6144) || wide);
+    if (cost < best_cost || tie) best = c.cfg, best_cost = cost;
   }
   return best;
 }
@@ -294,7 +298,7 @@ int rows_split(int64_t N, int64_t K) {
 template <int DT, int S, bool A4>
 hipError_t launch_rows_nb(const void* x, const uint8_t* wq, const float* ws, const float* bias, int64_t M, int64_t N,
                           int64_t K, void* out, const GatedResidual& gr, hipStream_t stream) {
-  switch (rows_split(N, K)) {
+  switch (rows_split(N, K, A4)) {
     case 16: return launch_rows_t<DT, S, A4, 1, 16, 3>(x, wq, ws, bias, M, N, K, out, gr, stream);
     case 1: return launch_rows_t<DT, S, A4, 1, 8, 3>(x, wq, ws, bias, M, N, K, out, gr, stream);
     case 2: return launch_rows_t<DT, S, A4, 2, 8, 3>(x, wq, ws, bias, M, N, K, out, gr, stream);
