@@ -558,12 +558,11 @@ def _gated_residual(residual: torch.Tensor, gate: torch.Tensor | None, out_shape
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 
 
-def _workspace(device: torch.device) -> torch.Tensor | None:
-    """The stream-K workspace of `device`'s current stream, or None under graph capture
-    before one exists (the W4A4 GEMM then runs a data-parallel plan, same results bit for
-    bit; the W4A16 GEMM its unsplit plan)."""
-    stream = torch.cuda.current_stream(device)
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream)
+def _workspace(device: torch.device, stream: int) -> torch.Tensor | None:
+    """The stream-K workspace of `device`'s current stream (its handle), or None under graph
+    capture before one exists (the W4A4 GEMM then runs a data-parallel plan, same results bit
+    for bit; the W4A16 GEMM its unsplit plan)."""
+    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     ws = _WORKSPACES.get(key)
     if ws is None:
         if torch.cuda.is_current_stream_capturing():
@@ -602,14 +601,15 @@ def _w4a4(act: torch.Tensor, act_format: int, k: int, qweight, xscales, wscales,
         out = gr.residual.view(m, n)
     else:
         out = torch.empty((m, n), dtype=output_dtype, device=act.device)
-    work = _workspace(act.device)
+    stream = torch.cuda.current_stream(act.device).cuda_stream  # once: an eager call is host time
+    work = _workspace(act.device, stream)
     nat.check(
         nat.load().convrot_w4a4_gemm_ws(
             nat.ptr(act), act_format, nat.ptr(xs), nat.ptr(w), nat.ptr(ws), nat.ptr(b), m, n, k,
             nat.ptr(gr.residual if gr is not None else None), nat.ptr(gr.gate if gr is not None else None),
             gr.stride if gr is not None else 0, gr.rows_per_gate if gr is not None else 1,
             nat.ptr(work), work.numel() if work is not None else 0,
-            nat.ptr(out), nat.dtype_code(output_dtype), nat.stream_of(act.device),
+            nat.ptr(out), nat.dtype_code(output_dtype), stream,
         )
     )
     return out
@@ -853,14 +853,15 @@ def hip_w4a16_matmul(activations, qweight, wscales, bias, *, output_dtype, out_f
     # the stream's W4A4 workspace lets the weight-streaming kernel split K over
     # workgroups (few output tiles, long K, M <= 32); none under graph capture
     # before it exists (the unsplit plan)
-    work = _workspace(act.device)
+    stream = torch.cuda.current_stream(act.device).cuda_stream
+    work = _workspace(act.device, stream)
     nat.check(
         nat.load().convrot_w4a16_gemm_ws(
             nat.ptr(act), nat.dtype_code(act.dtype), nat.ptr(w), nat.ptr(ws), nat.ptr(b), m, n, k,
             nat.ptr(gr.residual if gr is not None else None), nat.ptr(gr.gate if gr is not None else None),
             gr.stride if gr is not None else 0, gr.rows_per_gate if gr is not None else 1,
             nat.ptr(work), work.numel() if work is not None else 0,
-            nat.ptr(out), nat.dtype_code(output_dtype), nat.stream_of(act.device),
+            nat.ptr(out), nat.dtype_code(output_dtype), stream,
         )
     )
     return out
@@ -889,8 +890,8 @@ def _linear_rows_eligible(x2d: torch.Tensor, group_size: int, a4: bool) -> bool:
     """Whether ConvRotLinear runs these rows through convrot_linear_rows."""
     rows, features = x2d.shape
     max_rows, max_elements = LINEAR_ROWS_MAX[a4]
-    return (group_size in LINEAR_ROWS_GROUPS
-            and (rows == 1 or (1 < rows <= max_rows and rows * features <= max_elements))
+    return (0 < rows <= max_rows and (rows == 1 or rows * features <= max_elements)
+            and group_size in LINEAR_ROWS_GROUPS
             and x2d.dtype in ((torch.bfloat16, torch.float16, torch.float32) if a4
                               else (torch.bfloat16, torch.float16))
             and rows * features * x2d.element_size() <= LINEAR_ROWS_MAX_BYTES)
@@ -914,8 +915,7 @@ def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, 
     stream = torch.cuda.current_stream(device).cuda_stream
     # not used here: a program that warms a stream up with a few rows and then captures
     # more gets the plans that need the stream's workspace
-    if (device.index, stream) not in _WORKSPACES:
-        _workspace(device)
+    _workspace(device, stream)
     if gr is not None and gr.inplace:
         out = gr.residual.view(m, n)
         if _overlap(x2d, out):
