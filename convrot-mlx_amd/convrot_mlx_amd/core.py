@@ -915,7 +915,8 @@ def _linear_rows(x2d: torch.Tensor, group_size: int, a4: bool, w: torch.Tensor, 
     stream = torch.cuda.current_stream(device).cuda_stream
     # not used here: a program that warms a stream up with a few rows and then captures
     # more gets the plans that need the stream's workspace
-    _workspace(device, stream)
+    if (device.index, stream) not in _WORKSPACES:
+        _workspace(device, stream)
     if gr is not None and gr.inplace:
         out = gr.residual.view(m, n)
         if _overlap(x2d, out):
